@@ -33,7 +33,10 @@ struct Batch {
     DevOp *d_ops = nullptr;
     PJob *d_jobs = nullptr;
     double *d_results = nullptr;
-    int nitems = 0, ops_cap = 0, jobs_cap = 0;
+    // items by group (one launch each): group g holds items [first[g], first[g + 1]);
+    // groups[i] = partition i's
+    int nitems = 0, first[BATCH_GROUPS + 1] = {}, ops_cap = 0, jobs_cap = 0;
+    std::vector<int> groups;
     void *h_stage = nullptr;  // params | ops | jobs  (pinned)
     size_t stage_cap = 0;
     double *h_results = nullptr;
@@ -62,7 +65,8 @@ static int enqueue(Batch &b, int nparts, int tot_ops, int njobs) {
     if (ob) BHIP_TRY(hipMemcpyAsync(b.d_ops, (char *)b.h_stage + pb, ob, hipMemcpyHostToDevice, b.stream));
     if (jb) BHIP_TRY(hipMemcpyAsync(b.d_jobs, (char *)b.h_stage + pb + ob, jb, hipMemcpyHostToDevice, b.stream));
     BHIP_TRY(batch_pmatrix(b.prec, b.d_params, b.d_jobs, njobs, b.stream));
-    BHIP_TRY(batch_traverse(b.prec, b.d_params, b.d_items, b.nitems, b.grid, b.stream));
+    for (int g = 0; g < BATCH_GROUPS; g++)
+        BHIP_TRY(batch_traverse(b.prec, g, b.d_params, b.d_items + b.first[g], b.first[g + 1] - b.first[g], b.grid, b.stream));
     BHIP_TRY(hipMemcpyAsync(b.h_results, b.d_results, sizeof(double) * 2 * nparts, hipMemcpyDeviceToHost, b.stream));
     return PLK_OK;
 }
@@ -87,16 +91,49 @@ static int check_parts(plk_ctx *const *parts, int nparts, const char *who) {
     return PLK_OK;
 }
 
-// all tiles of all partitions, most expensive partitions first
-static std::vector<BatchItem> make_items(plk_ctx *const *parts, int nparts) {
+static int group_of(const plk_ctx &c) {
+    if (c.n == 4) return BATCH_4;
+    if (c.prec == PLK_FP64 && f64_form_of(c) == 1) return c.ncat > 1 ? BATCH_MC : BATCH_MC1;
+    return BATCH_20;
+}
+
+// Work items of all partitions by group, each group with its most expensive partitions first.
+static std::vector<BatchItem> make_items(Batch &b, plk_ctx *const *parts, int nparts) {
     std::vector<int> order(nparts);
     std::iota(order.begin(), order.end(), 0);
-    auto cost = [&](int i) { return (double)parts[i]->n * parts[i]->n * parts[i]->ntiles; };
-    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return cost(x) > cost(y); });
+    b.groups.resize(nparts);
+    for (int i = 0; i < nparts; i++) b.groups[i] = group_of(*parts[i]);
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
+        return b.groups[x] != b.groups[y] ? b.groups[x] < b.groups[y] : parts[x]->ntiles > parts[y]->ntiles;
+    });
     std::vector<BatchItem> items;
-    for (int i : order)
-        for (int t = 0; t < parts[i]->ntiles; t++) items.push_back(BatchItem{i, t});
+    std::fill(b.first, b.first + BATCH_GROUPS + 1, 0);
+    for (int i : order) {
+        const bool mc = b.groups[i] <= BATCH_MC1;
+        const int n = mc ? parts[i]->nptn_pad / mc_batch_patterns(parts[i]->ncat) : parts[i]->ntiles;
+        for (int t = 0; t < n; t++) items.push_back(BatchItem{i, t});
+        b.first[b.groups[i] + 1] = (int)items.size();
+    }
+    for (int g = 0; g < BATCH_GROUPS; g++) b.first[g + 1] = std::max(b.first[g + 1], b.first[g]);
     return items;
+}
+
+// Upload the items of `parts` (grown buffer; the stream is idle).
+static int upload_items(Batch &b, plk_ctx *const *parts, int nparts) {
+    const std::vector<BatchItem> items = make_items(b, parts, nparts);
+    b.nitems = 0;
+    if ((int)items.size() > b.items_cap) {
+        const int cap = std::max((int)items.size(), 2 * b.items_cap);
+        if (b.d_items) (void)hipFree(b.d_items);
+        b.d_items = nullptr;
+        b.items_cap = 0;
+        BHIP_TRY(hipMalloc((void **)&b.d_items, sizeof(BatchItem) * cap));
+        b.items_cap = cap;
+    }
+    BHIP_TRY(hipMemcpyAsync(b.d_items, items.data(), sizeof(BatchItem) * items.size(), hipMemcpyHostToDevice, b.stream));
+    BHIP_TRY(hipStreamSynchronize(b.stream));
+    b.nitems = (int)items.size();
+    return PLK_OK;
 }
 
 extern "C" int plk_batch_rebind(plk_batch *b, plk_ctx *const *parts, int nparts) {
@@ -107,7 +144,6 @@ extern "C" int plk_batch_rebind(plk_batch *b, plk_ctx *const *parts, int nparts)
     if (parts[0]->prec != b->prec) return fail(PLK_ERR_ARG, "plk_batch_rebind: the batch's precision form differs");
     BHIP_TRY(hipStreamSynchronize(b->stream));
     drop_graph(*b);
-    const std::vector<BatchItem> items = make_items(parts, nparts);
     if (nparts > b->parts_cap) {
         const int cap = std::max(nparts, 2 * b->parts_cap);
         // (plain hipFree/hipMalloc like plk_batch_create; growth doubles, so this is rare)
@@ -122,18 +158,9 @@ extern "C" int plk_batch_rebind(plk_batch *b, plk_ctx *const *parts, int nparts)
         BHIP_TRY(hipHostMalloc((void **)&b->h_results, sizeof(double) * 2 * cap, hipHostMallocDefault));
         b->parts_cap = cap;
     }
-    if ((int)items.size() > b->items_cap) {
-        const int cap = std::max((int)items.size(), 2 * b->items_cap);
-        if (b->d_items) (void)hipFree(b->d_items);
-        b->d_items = nullptr;
-        b->items_cap = 0;
-        BHIP_TRY(hipMalloc((void **)&b->d_items, sizeof(BatchItem) * cap));
-        b->items_cap = cap;
-    }
-    BHIP_TRY(hipMemcpyAsync(b->d_items, items.data(), sizeof(BatchItem) * items.size(), hipMemcpyHostToDevice, b->stream));
-    BHIP_TRY(hipStreamSynchronize(b->stream));
+    rc = upload_items(*b, parts, nparts);
+    if (rc) return rc;
     b->parts.assign(parts, parts + nparts);
-    b->nitems = (int)items.size();
     return PLK_OK;
 }
 
@@ -153,19 +180,16 @@ extern "C" int plk_batch_create(plk_batch **out, plk_ctx *const *parts, int npar
         plk_batch_destroy(b);
         return rc;
     };
-    const std::vector<BatchItem> items = make_items(parts, nparts);
-    b->nitems = (int)items.size();
     b->parts_cap = nparts;
-    b->items_cap = b->nitems;
     hipError_t e;
     if ((e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking)) != hipSuccess ||
         (e = hipMalloc(&b->d_params, sizeof(KParams) * nparts)) != hipSuccess ||
-        (e = hipMalloc(&b->d_items, sizeof(BatchItem) * items.size())) != hipSuccess ||
         (e = hipMalloc(&b->d_results, sizeof(double) * 2 * nparts)) != hipSuccess ||
         (e = hipHostMalloc((void **)&b->h_results, sizeof(double) * 2 * nparts, hipHostMallocDefault)) != hipSuccess ||
-        (e = hipEventCreate(&b->ev0)) != hipSuccess || (e = hipEventCreate(&b->ev1)) != hipSuccess ||
-        (e = hipMemcpy(b->d_items, items.data(), sizeof(BatchItem) * items.size(), hipMemcpyHostToDevice)) != hipSuccess)
+        (e = hipEventCreate(&b->ev0)) != hipSuccess || (e = hipEventCreate(&b->ev1)) != hipSuccess)
         return cleanup(fail(PLK_ERR_HIP, std::string("plk_batch_create: ") + hipGetErrorString(e)));
+    const int irc = upload_items(*b, parts, nparts);
+    if (irc) return cleanup(irc);
     *out = b;
     return PLK_OK;
 }
@@ -209,6 +233,14 @@ extern "C" int plk_batch_loglik(plk_batch *b, const int *a, const int *bref, con
             return fail(PLK_ERR_ARG, "plk_batch_loglik: bad branch for partition " + std::to_string(i));
         tot_ops += (int)c->pending.size();
         njobs += (int)c->jobs.size() + (b->prec == PLK_FP32 ? 1 : 0);
+    }
+    // a partition's kernel form was switched (plk_set_f64_form) since the items were made
+    bool same = b->nitems > 0;
+    for (int i = 0; i < nparts && same; i++) same = b->groups[i] == group_of(*b->parts[i]);
+    if (!same) {
+        drop_graph(*b);
+        const int rc = upload_items(*b, b->parts.data(), nparts);
+        if (rc) return rc;
     }
     const size_t pb = sizeof(KParams) * nparts, ob = sizeof(DevOp) * tot_ops, jb = sizeof(PJob) * njobs;
     if (pb + ob + jb > b->stage_cap) {

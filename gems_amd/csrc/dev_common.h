@@ -219,5 +219,33 @@ __device__ inline bool finish_tiles(const KParams &P, double v0, double v1, int 
     return s_last;
 }
 
+// finish_tiles for workgroups of nblk 16-pattern blocks: the first wavefront's lanes 0, 16, ...
+// hold the blocks' values.  The alignment's total is the sum over its 4 ntiles blocks in
+// index order, whatever the number of blocks per workgroup.
+__device__ inline void finish_blocks(const KParams &P, double v, int wg, int nblk) {
+    __shared__ int s_last16;
+    const int nblocks = 4 * P.ntiles;
+    if (threadIdx.x < 64) {
+        const int q = threadIdx.x >> 4;
+        if ((threadIdx.x & 15) == 0 && q < nblk) P.tile_sums[wg * nblk + q] = v;
+        __threadfence();
+        if (threadIdx.x == 0) s_last16 = atomicAdd(P.counter, 1u) == (unsigned)(nblocks / nblk) - 1;
+    }
+    __syncthreads();
+    if (s_last16 && threadIdx.x < 64) {
+        __threadfence();
+        double a = 0.0;
+        for (int i = threadIdx.x; i < nblocks; i += 64)
+            a += __hip_atomic_load(&P.tile_sums[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        a = wave_sum(a);
+        if (threadIdx.x == 0) {
+            P.result[0] = a;
+            P.result[1] = 0.0;
+            __hip_atomic_store(P.counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+    __syncthreads();
+}
+
 }  // namespace dev
 }  // namespace plk

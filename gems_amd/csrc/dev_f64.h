@@ -4,7 +4,7 @@
 // workgroup owns one tile and its wavefronts split the categories (wave w handles
 // c = w, w + nwaves, ...).  Element (ptn, c, x) of a partial is at
 // ((tile*ncat + c)*n + x)*64 + lane, so every load/store of one (c, x) by a wavefront
-// is one contiguous 512-byte segment.  All tiles are independent across the whole
+// is one contiguous 512-byte segment (20 states: eight 64-byte ones, see f64_xoff).  All tiles are independent across the whole
 // traversal (the reference's packets walk every node for their pattern slice,
 // tree/phylokernelnew.h:2851-2853), so one launch runs the full post-order op list with
 // no grid-wide barrier; each thread only re-reads values it wrote itself.
@@ -176,11 +176,20 @@ __device__ inline void pmatrix_f64_body(const KParams &P, const PJob &j, const i
         ex[c * n + i] = exp(P.eval[i] * (P.rates[c] * j.len));
     }
     __syncthreads();
-    // stored [c][i][x]: a column per i, x contiguous (matrix-core fragments and the
-    // column-at-a-time kernels read it that way)
-    for (int idx = threadIdx.x; idx < nc * n * n; idx += blockDim.x) {
-        const int c = cb + idx / (n * n), rem = idx % (n * n), x = rem / n, i = rem % n;
-        E[(int64_t)c * n * n + i * n + x] = P.evec[x * n + i] * ex[c * n + i];
+    // the 20-state matrix-core traversal takes the exponentials alone (and its leaf tables in
+    // mc_leaf order); otherwise echild is stored [c][i][x]: a column per i, x contiguous (the
+    // 61-state matrix-core fragments and the column-at-a-time kernels read it that way)
+    const bool frag = n == 20 && P.f64_form == 1;
+    if (frag) {
+        for (int idx = threadIdx.x; idx < nc * n; idx += blockDim.x) {
+            const int c = cb + idx / n, i = idx % n;
+            E[mc_leaf(ncat, c, i)] = ex[c * n + i];
+        }
+    } else {
+        for (int idx = threadIdx.x; idx < nc * n * n; idx += blockDim.x) {
+            const int c = cb + idx / (n * n), rem = idx % (n * n), x = rem / n, i = rem % n;
+            E[(int64_t)c * n * n + i * n + x] = P.evec[x * n + i] * ex[c * n + i];
+        }
     }
     if (j.leaf) {
         double *T = M + (int64_t)2 * ncat * n * n + (int64_t)j.side * (su + 1) * block;
@@ -205,9 +214,13 @@ __device__ inline void pmatrix_f64_body(const KParams &P, const PJob &j, const i
             }
 #pragma unroll
             for (int q = 0; q < 4; q++)
-                if (base + q * nt < total) T[(int64_t)ss[q] * block + cs[q] * n + xs[q]] = v[q];
+                if (base + q * nt < total)
+                    T[(int64_t)ss[q] * block + (frag ? mc_leaf(ncat, cs[q], xs[q]) : cs[q] * n + xs[q])] = v[q];
         }
-        for (int idx = threadIdx.x; idx < nc * n; idx += blockDim.x) T[(int64_t)su * block + cb * n + idx] = 1.0;
+        for (int idx = threadIdx.x; idx < nc * n; idx += blockDim.x) {
+            const int at = frag ? mc_leaf(ncat, cb + idx / n, idx % n) : cb * n + idx;
+            T[(int64_t)su * block + at] = 1.0;
+        }
     }
 }
 
@@ -367,7 +380,7 @@ __device__ __forceinline__ double op_partial_store(const KParams &P, const DevOp
             const double *__restrict__ R = part + (int64_t)op.right * P.slot_stride + off;
             double r[N];
 #pragma unroll
-            for (int i = 0; i < N; i++) r[i] = R[i * 64];
+            for (int i = 0; i < N; i++) r[i] = R[f64_xoff(N, i)];
 #pragma unroll
             for (int x = 0; x < N; x++) t[x] = 0.0;
 #pragma unroll
@@ -385,7 +398,7 @@ __device__ __forceinline__ double op_partial_store(const KParams &P, const DevOp
             const double *__restrict__ L = part + (int64_t)op.left * P.slot_stride + off;
             double l[N];
 #pragma unroll
-            for (int i = 0; i < N; i++) l[i] = L[i * 64];
+            for (int i = 0; i < N; i++) l[i] = L[f64_xoff(N, i)];
             constexpr int H = N / 2;
 #pragma unroll
             for (int h = 0; h < N; h += H) {
@@ -417,7 +430,7 @@ __device__ __forceinline__ double op_partial_store(const KParams &P, const DevOp
 #pragma unroll
         for (int x = 0; x < N; x++) o = fma(row[x], t[x], o);
         m = fmax(m, fabs(o));
-        dst[j * 64] = o;
+        dst[f64_xoff(N, j)] = o;
         __builtin_amdgcn_sched_barrier(0);
     }
     return m;
@@ -488,7 +501,7 @@ __device__ inline bool traverse_f64_body(const KParams &P, const int tile) {
             // one category per wavefront; the SAFE handling of the N <= 20 path below
             const int c = w;
             const bool mine = c < ncat;
-            const int64_t off = ((int64_t)tile * ncat + c) * N * 64 + lane;
+            const int64_t off = ((int64_t)tile * ncat + c) * N * 64 + f64_loff(N, lane);
             const int64_t a = p * ncat + c;
             unsigned sc = 0;
             if (P.safe && mine) {
@@ -500,7 +513,7 @@ __device__ inline bool traverse_f64_body(const KParams &P, const int tile) {
             if (P.safe && mine) {
                 if (op.kind != KIND_TT && m < kST && invar == 0.0) {
 #pragma unroll
-                    for (int j = 0; j < N; j++) outp[off + j * 64] *= kTwo256;
+                    for (int j = 0; j < N; j++) outp[off + f64_xoff(N, j)] *= kTwo256;
                     sc += 1;
                 }
                 scale[(int64_t)op.out_slot * P.scale_stride + a] = (uint16_t)sc;
@@ -508,7 +521,7 @@ __device__ inline bool traverse_f64_body(const KParams &P, const int tile) {
             wmax = m;
         }
         for (int c = w; c < (E61 ? 0 : ncat); c += ncw) {
-            const int64_t off = ((int64_t)tile * ncat + c) * N * 64 + lane;
+            const int64_t off = ((int64_t)tile * ncat + c) * N * 64 + f64_loff(N, lane);
             if constexpr (N <= 20) {
                 // SAFE: this category's children counts, also fetched ahead of the work
                 unsigned sc = 0;
@@ -523,7 +536,7 @@ __device__ inline bool traverse_f64_body(const KParams &P, const int tile) {
                     const int64_t a = p * ncat + c;
                     if (op.kind != KIND_TT && m < kST && invar == 0.0) {
 #pragma unroll
-                        for (int j = 0; j < N; j++) outp[off + j * 64] *= kTwo256;
+                        for (int j = 0; j < N; j++) outp[off + f64_xoff(N, j)] *= kTwo256;
                         sc += 1;
                     }
                     scale[(int64_t)op.out_slot * P.scale_stride + a] = (uint16_t)sc;
@@ -552,7 +565,7 @@ __device__ inline bool traverse_f64_body(const KParams &P, const int tile) {
             }
             wmax = fmax(wmax, m);
 #pragma unroll
-            for (int j = 0; j < N; j++) outp[off + j * 64] = out[j];
+            for (int j = 0; j < N; j++) outp[off + f64_xoff(N, j)] = out[j];
         }
         if (!P.safe) {
             // one check over all categories of the pattern (2019-2034, 1893-1907)
@@ -563,9 +576,9 @@ __device__ inline bool traverse_f64_body(const KParams &P, const int tile) {
             const bool do_scale = (op.kind != KIND_TT) && pm < kST && invar == 0.0;
             if (do_scale) {
                 for (int c = w; c < ncat; c += ncw) {
-                    const int64_t off = ((int64_t)tile * ncat + c) * N * 64 + lane;
+                    const int64_t off = ((int64_t)tile * ncat + c) * N * 64 + f64_loff(N, lane);
 #pragma unroll
-                    for (int j = 0; j < N; j++) outp[off + j * 64] *= kTwo256;
+                    for (int j = 0; j < N; j++) outp[off + f64_xoff(N, j)] *= kTwo256;
                 }
             }
             if (w == 0) scale[(int64_t)op.out_slot * P.scale_stride + p] = (uint16_t)(sc_norm + (do_scale ? 1u : 0u));
@@ -585,27 +598,28 @@ __device__ inline bool traverse_f64_body(const KParams &P, const int tile) {
     double *__restrict__ theta = (double *)P.theta;
 
     for (int c = w; c < ncat; c += ncw) {
-        const int64_t off = ((int64_t)tile * ncat + c) * N * 64 + lane;
+        const int64_t off = ((int64_t)tile * ncat + c) * N * 64 + f64_loff(N, lane);
         const double *__restrict__ v0 = s_val[0] + c * N;
         if (MODE == MODE_LOGL) {
             // lh_cat = sum_i val * node * dad (dotProduct3Vec 3044-3057; tip 2903-2914)
             double acc = 0.0;
 #pragma unroll
             for (int i = 0; i < N; i++) {
-                const double a = atip ? tip[i] : A[off + i * 64];
-                acc = fma(v0[i] * a, B[off + i * 64], acc);
+                const double a = atip ? tip[i] : A[off + f64_xoff(N, i)];
+                acc = fma(v0[i] * a, B[off + f64_xoff(N, i)], acc);
             }
             s_cat[0][c][lane] = acc;
         } else {
             // theta = node * dad (2187-2193; tip 2104-2145), then the triple dot (2499-2501)
             const double *__restrict__ v1 = s_val[1] + c * N;
             const double *__restrict__ v2 = s_val[2] + c * N;
+            const int64_t toff = ((int64_t)tile * ncat + c) * N * 64 + lane;
             double l0 = 0.0, l1 = 0.0, l2 = 0.0;
 #pragma unroll
             for (int i = 0; i < N; i++) {
-                const double a = atip ? tip[i] : A[off + i * 64];
-                const double th = a * B[off + i * 64];
-                if (theta) theta[off + i * 64] = th;  // null: derivatives only (many branches)
+                const double a = atip ? tip[i] : A[off + f64_xoff(N, i)];
+                const double th = a * B[off + f64_xoff(N, i)];
+                if (theta) theta[toff + i * 64] = th;  // null: derivatives only (many branches)
                 l0 = fma(v0[i], th, l0);
                 l1 = fma(v1[i], th, l1);
                 l2 = fma(v2[i], th, l2);
@@ -628,9 +642,9 @@ __device__ inline bool traverse_f64_body(const KParams &P, const int tile) {
                 const int d = s_sc[c][lane] - sc_min;
                 if (d != 0) {
                     const double f = safe_factor(d);
-                    const int64_t off = ((int64_t)tile * ncat + c) * N * 64 + lane;
+                    const int64_t toff = ((int64_t)tile * ncat + c) * N * 64 + lane;
 #pragma unroll
-                    for (int i = 0; i < N; i++) theta[off + i * 64] *= f;
+                    for (int i = 0; i < N; i++) theta[toff + i * 64] *= f;
                 }
             }
         }

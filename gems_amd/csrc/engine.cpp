@@ -76,6 +76,13 @@ int ensure_op_capacity(Ctx &c, int nops) {
     return PLK_OK;
 }
 
+// Measured per traversal: 61 states 3.06 -> 0.64 ms on the matrix cores (at most four
+// categories), 20 states 2.13 -> 1.31 ms (100 taxa x 49,994 patterns).
+int f64_form_of(const Ctx &c) {
+    if (!c.d_uinv_frag || (c.n == 61 && c.ncat > 4)) return 0;
+    return c.f64_form >= 0 ? c.f64_form : 1;
+}
+
 KParams make_params(Ctx &c) {
     KParams p{};
     p.n = c.n;
@@ -108,10 +115,7 @@ KParams make_params(Ctx &c) {
     p.piU = c.d_piU;
     p.tipvec = c.d_tipvec;
     p.uinv_frag = c.d_uinv_frag;
-    // measured per traversal: 61 states 3.06 -> 0.64 ms on the matrix cores; 20 states
-    // 2.22 ms vector ALU vs 2.61 ms matrix cores (rows padded 20 -> 32)
-    const int form = c.f64_form >= 0 ? c.f64_form : (c.n == 61 ? 1 : 0);
-    p.f64_form = (c.d_uinv_frag && c.ncat <= 4) ? form : 0;
+    p.f64_form = f64_form_of(c);
     p.ops = c.d_ops;
     p.nops = 0;
     p.ptn_lh = c.d_ptn_lh;
@@ -354,7 +358,7 @@ static int run_traversal(Ctx &c, KParams &p, int mode, bool used[3]) {
     std::vector<int32_t> perm;
     // (not for the 20-state FP32 traversal, which carries each op's output into the next
     // op of the list's own order)
-    const bool two_orders = !small && !(f32 && c.n == 20) && alt_order(c, c.pending, perm);
+    const bool two_orders = !small && !(c.n == 20 && (f32 || p.f64_form == 1)) && alt_order(c, c.pending, perm);
     bool inline_ops = false;
     SmallInline inl;
     p.perm = nullptr;
@@ -762,10 +766,16 @@ extern "C" int plk_set_model(plk_ctx *c, const double *eval, const double *evec,
     HIP_TRY(hipMemcpyAsync(c->d_model, m.data(), sizeof(double) * m.size(), hipMemcpyHostToDevice, c->stream));
     std::vector<double> uf;
     if (c->d_uinv_frag) {
-        // [rb][ks][lane] = U^-1[16 rb + lane % 16][4 ks + lane / 16], zero outside n x n
-        const int ks_n = (n + 3) / 4;
         uf.assign(mfma64_uinv_frag_size(n), 0.0);
-        for (size_t f = 0; f < uf.size(); f++) {
+        const int ks_n = (n + 3) / 4;
+        if (n == 20)
+            for (int x = 0; x < n; x++)
+                for (int i = 0; i < n; i++) {
+                    uf[mc_frag(x, i)] = inv_evec[x * n + i];
+                    uf[400 + mc_frag(x, i)] = evec[x * n + i];
+                }
+        // [rb][ks][lane] = U^-1[16 rb + lane % 16][4 ks + lane / 16], zero outside n x n
+        for (size_t f = 0; f < (n == 20 ? 0 : uf.size()); f++) {
             const int lane = (int)(f % 64), ks = (int)(f / 64) % ks_n, rb = (int)(f / 64) / ks_n;
             const int j = 16 * rb + lane % 16, x = 4 * ks + lane / 16;
             if (j < n && x < n) uf[f] = inv_evec[j * n + x];
@@ -1093,7 +1103,7 @@ extern "C" int plk_newton_multi(plk_ctx *c, int nbr, const int *a, const int *b,
         int round = std::min(6, std::max(limit, 1)), launched = 0;
         for (;;) {
             for (int k = 0; k < round; k++)
-                HIP_TRY(multi_newton(c->prec, ncw, (const KParams *)c->d_mparams, (const BatchItem *)c->d_mitems,
+                HIP_TRY(multi_newton(c->prec, c->n, ncw, (const KParams *)c->d_mparams, (const BatchItem *)c->d_mitems,
                                      nbr * c->ntiles, c->d_mnewton, c->stream));
             launched += round;
             HIP_TRY(hipMemcpyAsync(h, c->d_mnewton, sizeof(NewtonState) * nbr, hipMemcpyDeviceToHost, c->stream));
@@ -1166,7 +1176,8 @@ extern "C" int plk_get_partial(plk_ctx *c, int slot, double *partial, uint16_t *
                 const int cc = i / c->n, x = i % c->n;
                 const int64_t base = ((int64_t)(p / 64) * c->block + (int64_t)cc * c->n) * 64;
                 partial[(int64_t)p * c->block + i] =
-                    f32 ? raw[base + f32_xoff(c->n, x) + f32_loff(c->n, p % 64)] : raw[base + (int64_t)x * 64 + p % 64];
+                    f32 ? raw[base + f32_xoff(c->n, x) + f32_loff(c->n, p % 64)]
+                        : raw[base + f64_xoff(c->n, x) + f64_loff(c->n, p % 64)];
             }
     }
     if (scale && c->prec == PLK_FP32) return fail(PLK_ERR_ARG, "plk_get_partial: the FP32 form keeps exponents (plk_get_exponents)");
@@ -1346,7 +1357,7 @@ extern "C" int plk_branch_derivs_multi(plk_ctx *c, int nbr, const int *a, const 
     double *hres = (double *)((char *)c->h_stage + sizeof(KParams) * nbr);
     HIP_TRY(hipMemcpyAsync(c->d_mparams, c->h_stage, sizeof(KParams) * nbr, hipMemcpyHostToDevice, c->stream));
     timing_begin(*c, 2);
-    HIP_TRY(multi_derivs(c->prec, std::min(c->ncat, 4), (const KParams *)c->d_mparams, (const BatchItem *)c->d_mitems,
+    HIP_TRY(multi_derivs(c->prec, c->n, std::min(c->ncat, 4), (const KParams *)c->d_mparams, (const BatchItem *)c->d_mitems,
                          nbr * c->ntiles, c->stream));
     timing_end(*c, 2);
     HIP_TRY(hipMemcpyAsync(hres, c->d_mres, sizeof(double) * 2 * nbr, hipMemcpyDeviceToHost, c->stream));

@@ -18,8 +18,34 @@ constexpr int f32_ksteps(int n) { return (n + 3) / 4; }
 // FP32 leaf-table row length: the matrix-core forms pad a row to whole 16-row blocks
 // (zeros past n), so a lane's four output rows are one aligned 16-byte load
 constexpr int f32_trow(int n) { return n == 4 ? 4 : f32_xblocks(n) * 16; }
-// FP64 matrix-core traversal: U^-1 as A fragments [16-row block][4-state k step][lane]
-constexpr int mfma64_uinv_frag_size(int n) { return ((n + 15) / 16) * ((n + 3) / 4) * 64; }
+// FP64 matrix-core traversal, constant matrices as A fragments: 61 states U^-1
+// [16-row block][4-state k step][lane], 20 states U^-1 then U (mc_frag order)
+constexpr int mfma64_uinv_frag_size(int n) { return n == 20 ? 800 : ((n + 15) / 16) * ((n + 3) / 4) * 64; }
+// FP64 partial layout inside one (tile, category) block of 64 patterns.  20 states: groups of
+// 8 patterns, element (x, p) at ((p / 8) * 5 + x % 5) * 32 + (x / 5) * 8 + p % 8, so that the 16
+// lanes of the matrix-core traversal that share a category read or write 256 contiguous
+// bytes per k step; other state counts: element (x, p) at x * 64 + p.
+constexpr bool f64_rg(int n) { return n == 20; }
+__host__ __device__ constexpr int f64_xoff(int n, int x) { return f64_rg(n) ? (x % 5) * 32 + (x / 5) * 8 : x * 64; }
+__host__ __device__ constexpr int f64_loff(int n, int p) { return f64_rg(n) ? (p >> 3) * 160 + (p & 7) : p; }
+// FP64 matrix-core traversal of 20 states (dev_f64_cat.h): patterns of one wavefront, PG per
+// column; state 5 k + ks is k step ks of lane group k, row 5 i + xb is row i of tile row xb
+constexpr int mc_ncb(int ncat) { return ncat >= 3 ? 4 : ncat; }
+constexpr int mc_unit(int pg, int ncat) { return 4 * pg * (4 / mc_ncb(ncat)); }
+// place of M[x][i] in the fragments of a 20 x 20 matrix: per k step tile pairs [pair][k][i][2],
+// then tile row 4
+__host__ __device__ constexpr int mc_frag(int x, int i) {
+    const int xb = x % 5, al = (i / 5) * 4 + x / 5;
+    return (i % 5) * 80 + (xb < 4 ? (xb >> 1) * 32 + 2 * al + (xb & 1) : 64 + al);
+}
+// place of state x of category c in a leaf-table row or an op's exponentials (ncat x 20 doubles): per group of four
+// categories [k step pair][k][category][2], then k step 4, so that the lanes of one pattern
+// read contiguous 16-byte pieces
+__host__ __device__ constexpr int mc_leaf(int ncat, int c, int x) {
+    const int g = c >> 2, nb = ncat - 4 * g < 4 ? ncat - 4 * g : 4;
+    const int at = (x / 5) * nb + (c & 3), ks = x % 5;
+    return g * 80 + (ks < 4 ? (ks >> 1) * 8 * nb + 2 * at + (ks & 1) : 16 * nb + at);
+}
 // FP32 partial layout inside one (tile, category) block of 64 patterns.  20 states:
 // row groups of 4 states, element (x, p) at ((x / 4) * 64 + p) * 4 + x % 4, so the four
 // matrix-core output rows a lane holds (and the four B-operand rows it feeds) are one
@@ -232,15 +258,23 @@ constexpr size_t kSinkBytes = 8192;
 bool valid_ref(const Ctx &c, int r);
 int ensure_op_capacity(Ctx &c, int nops);
 
-// Batched partitions: one work item = one 64-pattern tile of one partition.
+// FP64 20 / 61 states: 1 matrix-core traversal, 0 vector-ALU kernels (engine.cpp)
+int f64_form_of(const Ctx &c);
+
+// Batched partitions: one work item = one workgroup's patterns of one partition: a 64-pattern
+// tile, or mc_batch_patterns patterns of an FP64 20-state one on the matrix cores.  Items are
+// launched in groups, one kernel each: matrix cores (several categories, one category),
+// 20 states, 4 states.
 struct BatchItem {
     int32_t part;
     int32_t tile;
 };
+enum : int { BATCH_MC = 0, BATCH_MC1 = 1, BATCH_20 = 2, BATCH_4 = 3, BATCH_GROUPS = 4 };
+constexpr int mc_batch_patterns(int ncat) { return 4 * mc_unit(ncat > 1 ? 2 : 1, ncat); }
 hipError_t batch_pmatrix(int prec, const KParams *params, const PJob *jobs, int njobs, hipStream_t s);
-hipError_t batch_traverse(int prec, const KParams *params, const BatchItem *items, int nitems, int grid,
+hipError_t batch_traverse(int prec, int group, const KParams *params, const BatchItem *items, int nitems, int grid,
                           hipStream_t s);
-hipError_t multi_derivs(int prec, int ncw, const KParams *params, const BatchItem *items, int nitems, hipStream_t s);
-hipError_t multi_newton(int prec, int ncw, const KParams *params, const BatchItem *items, int nitems,
+hipError_t multi_derivs(int prec, int n, int ncw, const KParams *params, const BatchItem *items, int nitems, hipStream_t s);
+hipError_t multi_newton(int prec, int n, int ncw, const KParams *params, const BatchItem *items, int nitems,
                         NewtonState *states, hipStream_t s);
 }  // namespace plk

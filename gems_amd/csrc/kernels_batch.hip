@@ -6,6 +6,7 @@
 // per-item branch, uniform within a workgroup).
 #include "dev_f32.h"
 #include "dev_f64.h"
+#include "dev_f64_cat.h"
 
 namespace plk {
 namespace {
@@ -43,49 +44,57 @@ __global__ void __launch_bounds__(256) k_batch_pmatrix_f32(const KParams *params
 
 // Persistent when gridDim < nitems: workgroup g takes items g, g + grid, ... (the host
 // orders items by decreasing cost, so the static stride is a longest-first schedule).
+// One kernel per state count: a kernel with both bodies takes the registers and LDS of the
+// larger one for every item (208 registers and 41 KB where DNA alone needs 57 and 19 KB).
+template <int N>
 __global__ void __launch_bounds__(256) k_batch_traverse_f64(const KParams *params, const BatchItem *items, int nitems) {
     for (int i = blockIdx.x; i < nitems; i += gridDim.x) {
         const BatchItem it = load_uniform(items + i);
         const KParams P = load_uniform(params + it.part);
-        if (P.n == 4) traverse_f64_body<4, MODE_LOGL>(P, it.tile);
-        else traverse_f64_body<20, MODE_LOGL>(P, it.tile);
+        traverse_f64_body<N, MODE_LOGL>(P, it.tile);
         __syncthreads();
     }
 }
 
+// the 20-state partitions of the matrix-core form: an item is one workgroup's patterns
+template <int PG>
+__global__ void __launch_bounds__(256, 2) k_batch_traverse_f64_cat(const KParams *params, const BatchItem *items, int nitems) {
+    for (int i = blockIdx.x; i < nitems; i += gridDim.x) {
+        const BatchItem it = load_uniform(items + i);
+        const KParams P = load_uniform(params + it.part);
+        traverse_f64_cat_body<MODE_LOGL, PG>(P, it.tile);
+        __syncthreads();
+    }
+}
+
+template <int N>
 __global__ void __launch_bounds__(256) k_batch_traverse_f32(const KParams *params, const BatchItem *items, int nitems) {
     for (int i = blockIdx.x; i < nitems; i += gridDim.x) {
         const BatchItem it = load_uniform(items + i);
         const KParams P = load_uniform(params + it.part);
-        if (P.n == 4) traverse_f32_valu_body<4, MODE_LOGL>(P, it.tile);
-        else traverse_f32_mfma_body<20, MODE_LOGL>(P, it.tile);
+        if constexpr (N == 4) traverse_f32_valu_body<4, MODE_LOGL>(P, it.tile);
+        else traverse_f32_mfma_body<N, MODE_LOGL>(P, it.tile);
         __syncthreads();
     }
 }
 
 // df/ddf of many branches of one alignment in one launch: item = (branch, tile); each
 // branch has its own KParams (branch ends, length, reduction buffers) and theta is not
-// stored.  Same arithmetic as the single-branch kernels, so results are identical.
-__global__ void __launch_bounds__(256) k_multi_derivs_f64(const KParams *params, const BatchItem *items, int nitems) {
+// stored.  Same arithmetic as the single-branch kernels, so results are identical.  One
+// kernel per state count (see above; with all three in one, every count ran with the
+// 61-state body's 512 registers, spills and 72 KB of LDS).
+template <int N>
+__global__ void __launch_bounds__(256) k_multi_derivs_f64(const KParams *params, const BatchItem *items) {
     const BatchItem it = load_uniform(items + blockIdx.x);
     const KParams P = load_uniform(params + it.part);
-    switch (P.n) {
-        case 4: traverse_f64_body<4, MODE_THETA>(P, it.tile); break;
-        case 20: traverse_f64_body<20, MODE_THETA>(P, it.tile); break;
-        case 61: traverse_f64_body<61, MODE_THETA>(P, it.tile); break;
-        default: break;
-    }
+    traverse_f64_body<N, MODE_THETA>(P, it.tile);
 }
 
-__global__ void __launch_bounds__(256) k_multi_derivs_f32(const KParams *params, const BatchItem *items, int nitems) {
+template <int N>
+__global__ void __launch_bounds__(256) k_multi_derivs_f32(const KParams *params, const BatchItem *items) {
     const BatchItem it = load_uniform(items + blockIdx.x);
     const KParams P = load_uniform(params + it.part);
-    switch (P.n) {
-        case 4: theta_f32_body<4>(P, it.tile); break;
-        case 20: theta_f32_body<20>(P, it.tile); break;
-        case 61: theta_f32_body<61>(P, it.tile); break;
-        default: break;
-    }
+    theta_f32_body<N>(P, it.tile);
 }
 
 // Many-branch Newton: item = (branch, tile); one launch = one derivative evaluation of
@@ -93,55 +102,56 @@ __global__ void __launch_bounds__(256) k_multi_derivs_f32(const KParams *params,
 // branch's minimizeNewton step in the workgroup finishing its reduction.  A finished
 // branch's items return at once.  (A branch's state is written only by its last
 // workgroup, after all of its items have read it.)
-__global__ void __launch_bounds__(256) k_multi_newton_f64(const KParams *params, const BatchItem *items,
-                                                          NewtonState *states) {
+template <int N, bool F32>
+__global__ void __launch_bounds__(256) k_multi_newton(const KParams *params, const BatchItem *items, NewtonState *states) {
     const BatchItem it = load_uniform(items + blockIdx.x);
     NewtonState *st = states + it.part;
     if (st->done) return;
     KParams P = load_uniform(params + it.part);
     P.br_len = st->rts;
-    bool last = false;
-    switch (P.n) {
-        case 4: last = traverse_f64_body<4, MODE_THETA, true>(P, it.tile); break;
-        case 20: last = traverse_f64_body<20, MODE_THETA, true>(P, it.tile); break;
-        case 61: last = traverse_f64_body<61, MODE_THETA, true>(P, it.tile); break;
-        default: break;
-    }
+    bool last;
+    if constexpr (F32) last = theta_f32_body<N, true>(P, it.tile);
+    else last = traverse_f64_body<N, MODE_THETA, true>(P, it.tile);
     if (last && threadIdx.x == 0) newton_record(*st, P.result[0], P.result[1], P.result[2]);
 }
 
-__global__ void __launch_bounds__(256) k_multi_newton_f32(const KParams *params, const BatchItem *items,
-                                                          NewtonState *states) {
-    const BatchItem it = load_uniform(items + blockIdx.x);
-    NewtonState *st = states + it.part;
-    if (st->done) return;
-    KParams P = load_uniform(params + it.part);
-    P.br_len = st->rts;
-    bool last = false;
-    switch (P.n) {
-        case 4: last = theta_f32_body<4, true>(P, it.tile); break;
-        case 20: last = theta_f32_body<20, true>(P, it.tile); break;
-        case 61: last = theta_f32_body<61, true>(P, it.tile); break;
-        default: break;
-    }
-    if (last && threadIdx.x == 0) newton_record(*st, P.result[0], P.result[1], P.result[2]);
+template <int N>
+void multi_newton_n(bool f32, int ncw, const KParams *params, const BatchItem *items, int nitems, NewtonState *states,
+                    hipStream_t s) {
+    if (f32) hipLaunchKernelGGL((k_multi_newton<N, true>), dim3(nitems), dim3(64 * ncw), 0, s, params, items, states);
+    else hipLaunchKernelGGL((k_multi_newton<N, false>), dim3(nitems), dim3(64 * ncw), 0, s, params, items, states);
+}
+
+template <int N>
+void multi_derivs_n(bool f32, int ncw, const KParams *params, const BatchItem *items, int nitems, hipStream_t s) {
+    if (f32) hipLaunchKernelGGL((k_multi_derivs_f32<N>), dim3(nitems), dim3(64 * ncw), 0, s, params, items);
+    else hipLaunchKernelGGL((k_multi_derivs_f64<N>), dim3(nitems), dim3(64 * ncw), 0, s, params, items);
 }
 
 }  // namespace
 
-hipError_t multi_newton(int prec, int ncw, const KParams *params, const BatchItem *items, int nitems,
+hipError_t multi_newton(int prec, int n, int ncw, const KParams *params, const BatchItem *items, int nitems,
                         NewtonState *states, hipStream_t s) {
     if (nitems <= 0) return hipSuccess;
-    if (prec == PLK_FP64)
-        hipLaunchKernelGGL(k_multi_newton_f64, dim3(nitems), dim3(64 * ncw), 0, s, params, items, states);
-    else hipLaunchKernelGGL(k_multi_newton_f32, dim3(nitems), dim3(64 * ncw), 0, s, params, items, states);
+    const bool f32 = prec == PLK_FP32;
+    switch (n) {
+        case 4: multi_newton_n<4>(f32, ncw, params, items, nitems, states, s); break;
+        case 20: multi_newton_n<20>(f32, ncw, params, items, nitems, states, s); break;
+        case 61: multi_newton_n<61>(f32, ncw, params, items, nitems, states, s); break;
+        default: return hipErrorInvalidValue;
+    }
     return hipGetLastError();
 }
 
-hipError_t multi_derivs(int prec, int ncw, const KParams *params, const BatchItem *items, int nitems, hipStream_t s) {
+hipError_t multi_derivs(int prec, int n, int ncw, const KParams *params, const BatchItem *items, int nitems, hipStream_t s) {
     if (nitems <= 0) return hipSuccess;
-    if (prec == PLK_FP64) hipLaunchKernelGGL(k_multi_derivs_f64, dim3(nitems), dim3(64 * ncw), 0, s, params, items, nitems);
-    else hipLaunchKernelGGL(k_multi_derivs_f32, dim3(nitems), dim3(64 * ncw), 0, s, params, items, nitems);
+    const bool f32 = prec == PLK_FP32;
+    switch (n) {
+        case 4: multi_derivs_n<4>(f32, ncw, params, items, nitems, s); break;
+        case 20: multi_derivs_n<20>(f32, ncw, params, items, nitems, s); break;
+        case 61: multi_derivs_n<61>(f32, ncw, params, items, nitems, s); break;
+        default: return hipErrorInvalidValue;
+    }
     return hipGetLastError();
 }
 
@@ -152,12 +162,22 @@ hipError_t batch_pmatrix(int prec, const KParams *params, const PJob *jobs, int 
     return hipGetLastError();
 }
 
-hipError_t batch_traverse(int prec, const KParams *params, const BatchItem *items, int nitems, int grid,
+hipError_t batch_traverse(int prec, int group, const KParams *params, const BatchItem *items, int nitems, int grid,
                           hipStream_t s) {
     if (nitems <= 0) return hipSuccess;
-    const int g = (grid <= 0 || grid > nitems) ? nitems : grid;
-    if (prec == PLK_FP64) hipLaunchKernelGGL(k_batch_traverse_f64, dim3(g), dim3(256), 0, s, params, items, nitems);
-    else hipLaunchKernelGGL(k_batch_traverse_f32, dim3(g), dim3(256), 0, s, params, items, nitems);
+    const dim3 g((grid <= 0 || grid > nitems) ? nitems : grid), b(256);
+    const bool f32 = prec == PLK_FP32;
+    switch (group) {
+        case BATCH_MC: hipLaunchKernelGGL(k_batch_traverse_f64_cat<2>, g, b, 0, s, params, items, nitems); break;
+        case BATCH_MC1: hipLaunchKernelGGL(k_batch_traverse_f64_cat<1>, g, b, 0, s, params, items, nitems); break;
+        case BATCH_20:
+            if (f32) hipLaunchKernelGGL(k_batch_traverse_f32<20>, g, b, 0, s, params, items, nitems);
+            else hipLaunchKernelGGL(k_batch_traverse_f64<20>, g, b, 0, s, params, items, nitems);
+            break;
+        default:
+            if (f32) hipLaunchKernelGGL(k_batch_traverse_f32<4>, g, b, 0, s, params, items, nitems);
+            else hipLaunchKernelGGL(k_batch_traverse_f64<4>, g, b, 0, s, params, items, nitems);
+    }
     return hipGetLastError();
 }
 

@@ -1,5 +1,6 @@
 // FP64 kernels for gfx950: thin __global__ wrappers over the bodies in dev_f64.h.
 #include "dev_f64.h"
+#include "dev_f64_cat.h"
 #include "dev_f64_mfma.h"
 
 namespace plk {
@@ -47,6 +48,34 @@ __global__ void __launch_bounds__(64 * MfmaShape<N>::RB, CSPLIT ? 4 : 2) k_trave
     }
 }
 
+// 20 states on the matrix cores; WIDE: 5-8 categories (two wavefronts per pattern unit).
+// PG = 2 takes 160 registers (three wavefronts per SIMD), PG = 1 119 (four).
+template <int MODE, int PG, bool WIDE>
+__global__ void __launch_bounds__(WIDE ? 512 : 256, 2) k_traverse_f64_cat(KParams P) {
+    traverse_f64_cat_body<MODE, PG>(P, blockIdx.x);
+}
+
+template <int MODE, int PG>
+void launch_cat(const KParams &p, hipStream_t s) {
+    const dim3 grid(p.nptn_pad / (4 * mc_unit(PG, p.ncat)));
+    if (p.ncat <= 4) hipLaunchKernelGGL((k_traverse_f64_cat<MODE, PG, false>), grid, dim3(256), 0, s, p);
+    else hipLaunchKernelGGL((k_traverse_f64_cat<MODE, PG, true>), grid, dim3(512), 0, s, p);
+}
+
+// PG = 1 while its wavefronts do not outnumber the SIMDs (4 patterns each: up to 4,096 patterns
+// with 3-4 categories on 256 compute units), where an op's latency is all that counts: 50
+// taxa x 3,855 patterns, all directions, 196 us against 270; beyond that PG = 2 has more
+// products in flight per wavefront and 64-byte pieces per row: 100 taxa x 6,000 patterns
+// 197 against 226 us, 24,000 577 against 798, 49,994 1.31 ms against 1.80.  One category
+// leaves no room for PG = 2 in a 64-pattern tile.
+template <int MODE>
+hipError_t traverse_cat(const KParams &p, hipStream_t s) {
+    const int waves = p.nptn_pad / mc_unit(1, p.ncat) * ((p.ncat + 3) / 4);
+    if (p.ncat > 1 && waves > 4 * p.ncu) launch_cat<MODE, 2>(p, s);
+    else launch_cat<MODE, 1>(p, s);
+    return hipGetLastError();
+}
+
 template <int N, int DERIV>
 __global__ void __launch_bounds__(256) k_theta_eval_f64(KParams P) {
     theta_eval_f64_body<N, DERIV>(P, blockIdx.x, P.br_len);
@@ -72,8 +101,20 @@ template <int N>
 hipError_t traverse_n(const KParams &p0, int mode, hipStream_t s) {
     KParams p = p0;
     dim3 grid(p.ntiles), block(64 * p.ncw);
-    if constexpr (N != 4) {
-        if (p.f64_form == 1 && p.ncat <= 4 && p.uinv_frag) {
+    if constexpr (N == 20) {
+        if (p.f64_form == 1) {
+            if (mode == MODE_LOGL) return traverse_cat<MODE_LOGL>(p, s);
+            if (p.nops > 0) {
+                const hipError_t e = traverse_cat<MODE_PARTIALS>(p, s);
+                if (e != hipSuccess || mode == MODE_PARTIALS) return e;
+            } else if (mode == MODE_PARTIALS) {
+                return hipSuccess;
+            }
+            p.nops = 0;  // theta in the vector kernel, without ops
+        }
+    }
+    if constexpr (N == 61) {
+        if (p.f64_form == 1) {
             // the op list on the matrix cores, then the branch stage alone (no ops) in the
             // vector kernel
             if (p.nops > 0) {

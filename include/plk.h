@@ -21,9 +21,10 @@
  *   - A "node reference" is a slot id (>= 0) holding a directional partial, or a tip,
  *     encoded as -(taxon+1).
  *   - Partials use IQ-TREE's eigen-space representation in the FP64 form
- *     (tree/phylokernelnew.h:1989-1994) and are laid out on the device exactly like
- *     the reference's SIMD layout with 64 lanes: element (ptn, c, x) at
- *     (floor(ptn/64)*block + c*n + x)*64 + ptn%64, block = ncat*n.
+ *     (tree/phylokernelnew.h:1989-1994) and are laid out on the device like the
+ *     reference's SIMD layout with 64 lanes: element (ptn, c, x) at
+ *     (floor(ptn/64)*block + c*n + x)*64 + ptn%64, block = ncat*n (20 states: inside the
+ *     64-pattern block of a category, groups of 8 patterns, see f64_xoff/f64_loff).
  *   - scale counts follow scale_num (tree/phylonode.h:17, uint16): one per pattern in
  *     NORM mode, one per (pattern, category) in SAFE mode
  *     (tree/phylokernelnew.h:1924-1936, mode rule tree/phylotreesse.cpp:95-96).
@@ -171,11 +172,11 @@ int plk_get_exponents(plk_ctx *ctx, int slot, int32_t *exponents);
  * parallelism; fewer reuse each matrix fragment over more patterns).  Results do not
  * depend on it. */
 int plk_set_tile_shape(plk_ctx *ctx, int waves_per_category);
-/* FP64 contexts with 20 or 61 states and at most four categories: form 1 runs the
- * partial-likelihood ops on the matrix cores (FP64 16x16x4 tiles, one workgroup per 16
- * patterns); form 0 the vector-ALU kernels; -1 (default) picks by state count, the faster
- * one measured (61 states: matrix cores, 20: vector ALU).  Same results to rounding (the
- * sums run in a different order); scale counts follow the same rule. */
+/* FP64 contexts with 20 states, or 61 states and at most four categories: form 1 runs the
+ * partial-likelihood ops on the matrix cores (20 states: 4x4x4 tiles, four categories in one
+ * wavefront; 61: 16x16x4 tiles, one workgroup per 16 patterns); form 0 the vector-ALU
+ * kernels; -1 (default) the faster one measured, the matrix cores for both.  Same results
+ * to rounding (the sums run in a different order); scale counts follow the same rule. */
 /* Side outputs of the last plk_branch_loglik (FP64 form), as computeLikelihoodBranch
  * leaves them: lh_cat[p * ncat + c] = the category's likelihood w_c * sum_i val * node * dad
  * in the pattern's scaled frame, SAFE categories above the minimum count scaled by 2^-256

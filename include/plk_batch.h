@@ -4,8 +4,8 @@
  * IQ-TREE evaluates a partitioned analysis by looping over per-partition PhyloTrees
  * (PhyloSuperTree::computeLikelihood, tree/phylosupertree.cpp:709-734, OpenMP over
  * partitions ordered by cost, :662-707).  A batch runs that loop as ONE P(t) launch plus
- * ONE persistent traversal launch over all partitions' 64-pattern tiles, replayed as a
- * HIP graph while the launch shape is unchanged.  Each partition is a plk_ctx whose ops
+ * one persistent traversal launch per kernel (4 states, 20 states) over all partitions'
+ * pattern tiles, replayed as a HIP graph while the launch shape is unchanged.  Each partition is a plk_ctx whose ops
  * were queued with plk_update_partials; results per partition are bit-identical to
  * evaluating that context alone.
  */
