@@ -37,6 +37,7 @@ struct Batch {
     // groups[i] = partition i's
     int nitems = 0, first[BATCH_GROUPS + 1] = {}, ops_cap = 0, jobs_cap = 0;
     std::vector<int> groups;
+    size_t lds = 0;  // dynamic LDS of the 4-state launch
     void *h_stage = nullptr;  // params | ops | jobs  (pinned)
     size_t stage_cap = 0;
     double *h_results = nullptr;
@@ -44,7 +45,8 @@ struct Batch {
     bool use_graph = true;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
-    int g_ops = -1, g_jobs = -1, g_grid = -1;  // launch shape captured in the graph
+    int g_ops = -1, g_jobs = -1, g_grid = -1, g_dna = -1;
+    size_t g_lds = 0;  // launch shape captured in the graph
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     double t_total = 0.0;
     int64_t t_count = 0, updates = 0;
@@ -59,14 +61,17 @@ static void drop_graph(Batch &b) {
 }
 
 // Enqueue the whole batch evaluation on b.stream (captured into the graph when enabled).
-static int enqueue(Batch &b, int nparts, int tot_ops, int njobs) {
+static int enqueue(Batch &b, int nparts, int tot_ops, int njobs, int ndna) {
     const size_t pb = sizeof(KParams) * nparts, ob = sizeof(DevOp) * tot_ops, jb = sizeof(PJob) * njobs;
     BHIP_TRY(hipMemcpyAsync(b.d_params, b.h_stage, pb, hipMemcpyHostToDevice, b.stream));
     if (ob) BHIP_TRY(hipMemcpyAsync(b.d_ops, (char *)b.h_stage + pb, ob, hipMemcpyHostToDevice, b.stream));
     if (jb) BHIP_TRY(hipMemcpyAsync(b.d_jobs, (char *)b.h_stage + pb + ob, jb, hipMemcpyHostToDevice, b.stream));
-    BHIP_TRY(batch_pmatrix(b.prec, b.d_params, b.d_jobs, njobs, b.stream));
+    // the jobs of the 4-state traversal (dev_dna.h) come first
+    BHIP_TRY(batch_pmatrix_dna(b.prec, b.d_params, b.d_jobs, ndna, b.stream));
+    BHIP_TRY(batch_pmatrix(b.prec, b.d_params, b.d_jobs + ndna, njobs - ndna, b.stream));
     for (int g = 0; g < BATCH_GROUPS; g++)
-        BHIP_TRY(batch_traverse(b.prec, g, b.d_params, b.d_items + b.first[g], b.first[g + 1] - b.first[g], b.grid, b.stream));
+        BHIP_TRY(batch_traverse(b.prec, g, b.d_params, b.d_items + b.first[g], b.first[g + 1] - b.first[g], b.grid, b.lds,
+                                b.stream));
     BHIP_TRY(hipMemcpyAsync(b.h_results, b.d_results, sizeof(double) * 2 * nparts, hipMemcpyDeviceToHost, b.stream));
     return PLK_OK;
 }
@@ -92,7 +97,7 @@ static int check_parts(plk_ctx *const *parts, int nparts, const char *who) {
 }
 
 static int group_of(const plk_ctx &c) {
-    if (c.n == 4) return BATCH_4;
+    if (c.n == 4) return !dna_form(c) ? BATCH_4 : c.prec == PLK_FP64 && c.safe ? BATCH_DNA_SAFE : BATCH_DNA;
     if (c.prec == PLK_FP64 && f64_form_of(c) == 1) return c.ncat > 1 ? BATCH_MC : BATCH_MC1;
     return BATCH_20;
 }
@@ -224,7 +229,7 @@ extern "C" int plk_batch_loglik(plk_batch *b, const int *a, const int *bref, con
     if (!b || !a || !bref || !t) return fail(PLK_ERR_ARG, "plk_batch_loglik: null argument");
     const int nparts = (int)b->parts.size();
     // --- per-partition validation and op/job gathering (the queued ops of each context)
-    int tot_ops = 0, njobs = 0;
+    int tot_ops = 0, njobs = 0, ndna = 0;
     for (int i = 0; i < nparts; i++) {
         plk_ctx *c = b->parts[i];
         if (!c->model_set || !c->patterns_set) return fail(PLK_ERR_STATE, "plk_batch_loglik: partition not initialised");
@@ -232,7 +237,9 @@ extern "C" int plk_batch_loglik(plk_batch *b, const int *a, const int *bref, con
         if (!valid_ref(*c, ra) || !valid_ref(*c, rb) || (ra < 0 && rb < 0) || ra == rb || !std::isfinite(t[i]) || t[i] < 0)
             return fail(PLK_ERR_ARG, "plk_batch_loglik: bad branch for partition " + std::to_string(i));
         tot_ops += (int)c->pending.size();
-        njobs += (int)c->jobs.size() + (b->prec == PLK_FP32 ? 1 : 0);
+        const int nj = (int)c->jobs.size() + (b->prec == PLK_FP32 ? 1 : 0);
+        njobs += nj;
+        if (dna_form(*c)) ndna += nj;
     }
     // a partition's kernel form was switched (plk_set_f64_form) since the items were made
     bool same = b->nitems > 0;
@@ -269,7 +276,8 @@ extern "C" int plk_batch_loglik(plk_batch *b, const int *a, const int *bref, con
     KParams *hp = (KParams *)b->h_stage;
     DevOp *hop = (DevOp *)((char *)b->h_stage + pb);
     PJob *hj = (PJob *)((char *)b->h_stage + pb + ob);
-    int op_off = 0, job_off = 0;
+    int op_off = 0, dna_off = 0, other_off = ndna;
+    b->lds = 0;
     for (int i = 0; i < nparts; i++) {
         plk_ctx *c = b->parts[i];
         const int nops = (int)c->pending.size();
@@ -277,7 +285,13 @@ extern "C" int plk_batch_loglik(plk_batch *b, const int *a, const int *bref, con
         if (rc) return rc;
         int ra = a[i], rb = bref[i];
         if (rb < 0) std::swap(ra, rb);
+        const bool dna = dna_form(*c);
+        int &job_off = dna ? dna_off : other_off;
         KParams p = make_params(*c);
+        if (dna) {
+            p.nbuf = plan_dna(c->nslots, c->pending, {0, nops}, dna_max_buf(b->nitems, c->ncu));
+            b->lds = std::max(b->lds, dna_lds_bytes(b->prec == PLK_FP32 ? 1 : 0, c->ncat, 4, p.nbuf, 0, 0));
+        }
         p.ops = b->d_ops + op_off;
         p.nops = nops;
         p.mats = c->d_mats;
@@ -297,14 +311,15 @@ extern "C" int plk_batch_loglik(plk_batch *b, const int *a, const int *bref, con
         c->theta_valid = false;
     }
     // --- launch: graph replay when the captured launch shape still applies
-    const bool replay = b->use_graph && b->exec && b->g_ops == tot_ops && b->g_jobs == njobs && b->g_grid == b->grid;
+    const bool replay = b->use_graph && b->exec && b->g_ops == tot_ops && b->g_jobs == njobs && b->g_grid == b->grid && b->g_dna == ndna &&
+                        b->g_lds == b->lds;
     BHIP_TRY(hipEventRecord(b->ev0, b->stream));
     if (replay) {
         BHIP_TRY(hipGraphLaunch(b->exec, b->stream));
     } else if (b->use_graph) {
         drop_graph(*b);
         BHIP_TRY(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-        int rc = enqueue(*b, nparts, tot_ops, njobs);
+        int rc = enqueue(*b, nparts, tot_ops, njobs, ndna);
         hipGraph_t g = nullptr;
         hipError_t ce = hipStreamEndCapture(b->stream, &g);
         if (rc) {
@@ -317,9 +332,11 @@ extern "C" int plk_batch_loglik(plk_batch *b, const int *a, const int *bref, con
         b->g_ops = tot_ops;
         b->g_jobs = njobs;
         b->g_grid = b->grid;
+        b->g_dna = ndna;
+        b->g_lds = b->lds;
         BHIP_TRY(hipGraphLaunch(b->exec, b->stream));
     } else {
-        int rc = enqueue(*b, nparts, tot_ops, njobs);
+        int rc = enqueue(*b, nparts, tot_ops, njobs, ndna);
         if (rc) return rc;
     }
     BHIP_TRY(hipEventRecord(b->ev1, b->stream));

@@ -666,19 +666,19 @@ __device__ inline void traverse_f32_valu_body(const KParams &P, const int tile) 
         for (int ci = 0; ci < CPW; ci++) {
             const int c = w + ci * ncw;
             if (c >= ncat) break;
-            const int64_t off = ((int64_t)tile * ncat + c) * N * 64 + lane;
+            const int64_t off = ((int64_t)tile * ncat + c) * N * 64 + f32_loff(N, lane);
             const cfptr PL = as_constf(M + (int64_t)c * FR);
             const cfptr PR = as_constf(M + (int64_t)(ncat + c) * FR);
             float l[N], r[N];
             if (op.kind == KIND_II) {
                 const float *__restrict__ L = part + (int64_t)op.left * P.slot_stride + off;
 #pragma unroll
-                for (int y = 0; y < N; y++) l[y] = L[y * 64];
+                for (int y = 0; y < N; y++) l[y] = L[f32_xoff(N, y)];
             }
             if (op.kind != KIND_TT) {
                 const float *__restrict__ R = part + (int64_t)op.right * P.slot_stride + off;
 #pragma unroll
-                for (int y = 0; y < N; y++) r[y] = R[y * 64];
+                for (int y = 0; y < N; y++) r[y] = R[f32_xoff(N, y)];
             }
             const float *tl = tabs + ((int64_t)sl * ncat + c) * N;
             const float *tr = tabs + (int64_t)(P.su + 1) * ncat * N + ((int64_t)sr * ncat + c) * N;
@@ -713,9 +713,9 @@ __device__ inline void traverse_f32_valu_body(const KParams &P, const int tile) 
         for (int ci = 0; ci < CPW; ci++) {
             const int c = w + ci * ncw;
             if (c >= ncat) break;
-            const int64_t off = ((int64_t)tile * ncat + c) * N * 64 + lane;
+            const int64_t off = ((int64_t)tile * ncat + c) * N * 64 + f32_loff(N, lane);
 #pragma unroll
-            for (int x = 0; x < N; x++) outp[off + x * 64] = ldexpf(out[ci][x], -e);
+            for (int x = 0; x < N; x++) outp[off + f32_xoff(N, x)] = ldexpf(out[ci][x], -e);
         }
         if (w == 0) {
             int es = e;
@@ -731,20 +731,20 @@ __device__ inline void traverse_f32_valu_body(const KParams &P, const int tile) 
     const bool atip = P.br_a < 0;
     const int sa = atip ? P.states[(int64_t)(-P.br_a - 1) * P.nptn_pad + p] : 0;
     for (int c = w; c < ncat; c += ncw) {
-        const int64_t off = ((int64_t)tile * ncat + c) * N * 64 + lane;
+        const int64_t off = ((int64_t)tile * ncat + c) * N * 64 + f32_loff(N, lane);
         const cfptr Pt = as_constf(Mt + (int64_t)c * FR);
         const float *__restrict__ B = (const float *)P.part + (int64_t)P.br_b * P.slot_stride + off;
         const float *__restrict__ A = (const float *)P.part + (int64_t)(atip ? 0 : P.br_a) * P.slot_stride + off;
         float b[N];
 #pragma unroll
-        for (int y = 0; y < N; y++) b[y] = B[y * 64];
+        for (int y = 0; y < N; y++) b[y] = B[f32_xoff(N, y)];
         float acc = 0.0f;
 #pragma unroll
         for (int x = 0; x < N; x++) {
             float d = 0.0f;
 #pragma unroll
             for (int y = 0; y < N; y++) d = fmaf(Pt[x * N + y], b[y], d);
-            const float a = atip ? (float)P.tipvec[sa * N + x] : A[x * 64];
+            const float a = atip ? (float)P.tipvec[sa * N + x] : A[f32_xoff(N, x)];
             acc = fmaf((float)P.pi[x] * a, d, acc);
         }
         s_cat[c][lane] = (double)acc;

@@ -19,7 +19,7 @@
 // (the sums the leaf tables hold, in the same order), so no op waits on memory other
 // than its children.
 //
-// Layout of one LDS partial buffer: [c][x][lane] reals (the HBM layout of one tile).
+// Layout of one LDS partial buffer: the HBM layout of one tile.
 #pragma once
 
 #include "dev_common.h"
@@ -68,15 +68,22 @@ __device__ __forceinline__ SmallLds<REAL> small_lds(const KParams &P, char *base
     return s;
 }
 
+// Place of a lane's pattern and step from state to state in a (tile, category) block, in LDS
+// as in HBM (FP64 [state][pattern], FP32 [pattern][state]).
+template <typename REAL>
+__device__ __forceinline__ constexpr int small_off(int lane) { return sizeof(REAL) == 8 ? lane : lane * 4; }
+template <typename REAL>
+__device__ __forceinline__ constexpr int small_step() { return sizeof(REAL) == 8 ? 64 : 1; }
+
 // One category's 4 values of a child partial (LDS buffer or HBM).
 template <typename REAL>
 __device__ __forceinline__ void small_child_vals(const KParams &P, const SmallLds<REAL> &L, int ref, int lds, int c,
                                                  int tile, int lane, REAL (&v)[4]) {
-    const REAL *src = lds >= 0 ? L.part + ((size_t)lds * P.ncat + c) * 4 * 64 + lane
+    const REAL *src = lds >= 0 ? L.part + ((size_t)lds * P.ncat + c) * 4 * 64 + small_off<REAL>(lane)
                                : (const REAL *)P.part + (int64_t)ref * P.slot_stride +
-                                     ((int64_t)tile * P.ncat + c) * 4 * 64 + lane;
+                                     ((int64_t)tile * P.ncat + c) * 4 * 64 + small_off<REAL>(lane);
 #pragma unroll
-    for (int i = 0; i < 4; i++) v[i] = src[i * 64];
+    for (int i = 0; i < 4; i++) v[i] = src[i * small_step<REAL>()];
 }
 
 __device__ __forceinline__ int small_tip_state(const KParams &P, const uint8_t *staged, int taxon, int idx, int tile,
@@ -389,15 +396,15 @@ __device__ inline void traverse_small_body(const KParams &P, const int tile, cha
                 for (int ci = 0; ci < CPW; ci++) {
                     const int c = cw + ci * CW;
                     if (c >= ncat) break;
-                    REAL *dst = (REAL *)P.part + (int64_t)op.out_slot * P.slot_stride + ((int64_t)tile * ncat + c) * 4 * 64 + lane;
-                    REAL *lb = op.lds_out >= 0 ? L.part + ((size_t)op.lds_out * ncat + c) * 4 * 64 + lane : nullptr;
+                    REAL *dst = (REAL *)P.part + (int64_t)op.out_slot * P.slot_stride + ((int64_t)tile * ncat + c) * 4 * 64 + small_off<REAL>(lane);
+                    REAL *lb = op.lds_out >= 0 ? L.part + ((size_t)op.lds_out * ncat + c) * 4 * 64 + small_off<REAL>(lane) : nullptr;
 #pragma unroll
                     for (int j = 0; j < 4; j++) {
                         REAL v;
                         if constexpr (FORM == 0) v = do_scale ? out[ci][j] * kTwo256 : out[ci][j];
                         else v = ldexpf(out[ci][j], -e);
-                        dst[j * 64] = v;
-                        if (lb) lb[j * 64] = v;
+                        dst[j * small_step<REAL>()] = v;
+                        if (lb) lb[j * small_step<REAL>()] = v;
                     }
                 }
             }

@@ -40,7 +40,9 @@ static bool supported_states(int n) { return n == 4 || n == 20 || n == 61; }
 static int64_t mat_stride_of(int n, int ncat, int su, int prec) {
     if (prec == PLK_FP32) {
         int64_t fr = (int64_t)f32_xblocks(n) * f32_ksteps(n) * 64;
-        return round_up(2LL * ncat * fr + 2LL * (su + 1) * f32_trow(n) * ncat, 64);
+        int64_t len = 2LL * ncat * fr + 2LL * (su + 1) * f32_trow(n) * ncat;
+        if (n == 4) len = std::max<int64_t>(len, 2LL * dna_side_len(1, (ncat + 3) / 4));
+        return round_up(len, 64);
     }
     return round_up(2LL * ncat * n * n + 2LL * (su + 1) * n * ncat, 32);
 }
@@ -290,6 +292,97 @@ static void plan_small(Ctx &c, bool branch, int br_a, int br_b, SmallPlan &sp) {
     if (sp.stage) sp.lds_bytes = ((sp.lds_bytes + 15) & ~(size_t)15) + stage;
 }
 
+// Ops that touch a slot some op of the list writes depend on each other; all others are
+// independent, e.g. the ops of different NNI candidates.
+std::vector<int32_t> split_ops(int nslots, std::vector<DevOp> &ops, int max_ranges, std::vector<int> &newpos) {
+    const int n = (int)ops.size();
+    newpos.resize(n);
+    std::iota(newpos.begin(), newpos.end(), 0);
+    if (max_ranges <= 1 || n <= 1) return {0, n};
+    std::vector<int> parent(n), owner(nslots, -1);
+    std::iota(parent.begin(), parent.end(), 0);
+    auto find = [&](int x) {
+        while (parent[x] != x) x = parent[x] = parent[parent[x]];
+        return x;
+    };
+    for (int i = 0; i < n; i++) {
+        const int s = ops[i].out_slot;
+        if (owner[s] < 0) owner[s] = i;
+        else parent[find(i)] = find(owner[s]);
+    }
+    for (int i = 0; i < n; i++) {
+        if (ops[i].kind == KIND_II && owner[ops[i].left] >= 0) parent[find(i)] = find(owner[ops[i].left]);
+        if (ops[i].kind != KIND_TT && owner[ops[i].right] >= 0) parent[find(i)] = find(owner[ops[i].right]);
+    }
+    // components in order of their first op, each in list order
+    std::vector<int> comp(n), rank(n, -1), order(n);
+    int nc = 0;
+    for (int i = 0; i < n; i++) {
+        const int r = find(i);
+        if (rank[r] < 0) rank[r] = nc++;
+        comp[i] = rank[r];
+    }
+    if (nc <= 1) return {0, n};
+    std::iota(order.begin(), order.end(), 0);
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return comp[a] < comp[b]; });
+    std::vector<DevOp> sorted(n);
+    for (int i = 0; i < n; i++) {
+        sorted[i] = ops[order[i]];
+        newpos[order[i]] = i;
+    }
+    ops.swap(sorted);
+    // a range ends at a component's end once it holds its share of the ops
+    const int ranges = std::min(nc, max_ranges);
+    std::vector<int32_t> first{0};
+    for (int i = 0; i < n; i++) {
+        const bool end = i + 1 == n || comp[order[i]] != comp[order[i + 1]];
+        if (end && ((int64_t)(i + 1) * ranges >= (int64_t)n * (int64_t)first.size() || i + 1 == n)) first.push_back(i + 1);
+    }
+    return first;
+}
+
+int plan_dna(int nslots, std::vector<DevOp> &ops, const std::vector<int32_t> &first, int max_buf) {
+    int used = 0;
+    std::vector<int> current(nslots, -1), last(ops.size(), -1), prod_l(ops.size(), -1), prod_r(ops.size(), -1);
+    for (size_t q = 0; q + 1 < first.size(); q++) {
+        // reads of values that an earlier op but the previous one left (that one is in registers)
+        for (int i = first[q]; i < first[q + 1]; i++) {
+            DevOp &o = ops[i];
+            o.lds_left = o.lds_right = o.lds_out = -1;
+            if (o.kind == KIND_II) prod_l[i] = current[o.left];
+            if (o.kind != KIND_TT) prod_r[i] = current[o.right];
+            for (int v : {prod_l[i], prod_r[i]})
+                if (v >= 0 && v != i - 1) last[v] = i;
+            current[o.out_slot] = i;
+        }
+        std::vector<int> holder(max_buf, -1);  // value in each buffer
+        auto buffer_of = [&](int v) {
+            for (int b = 0; b < max_buf; b++)
+                if (v >= 0 && holder[b] == v) return b;
+            return -1;
+        };
+        for (int i = first[q]; i < first[q + 1]; i++) {
+            DevOp &o = ops[i];
+            if (prod_l[i] != i - 1) o.lds_left = buffer_of(prod_l[i]);
+            if (prod_r[i] != i - 1) o.lds_right = buffer_of(prod_r[i]);
+            if (last[i] <= i) continue;
+            // a free buffer, one whose value is done, or the one needed last if that is later
+            int at = -1;
+            for (int b = 0; b < max_buf && at < 0; b++)
+                if (holder[b] < 0 || last[holder[b]] <= i) at = b;
+            if (at < 0)
+                for (int b = 0; b < max_buf; b++)
+                    if (last[holder[b]] > last[i] && (at < 0 || last[holder[b]] > last[holder[at]])) at = b;
+            if (at < 0) continue;
+            holder[at] = i;
+            o.lds_out = at;
+            used = std::max(used, at + 1);
+        }
+        for (int i = first[q]; i < first[q + 1]; i++) current[ops[i].out_slot] = -1;
+    }
+    return used;
+}
+
 // Upload the queued ops, run the P(t) kernel, then one traversal launch in `mode`.
 // The FP32 form also needs P(t) of the branch itself (an extra job after the ops) for
 // the logL stage, and computes theta in a separate FP64 kernel after the traversal.
@@ -347,25 +440,59 @@ static int run_traversal(Ctx &c, KParams &p, int mode, bool used[3]) {
     p.ops = c.d_ops;
     p.mats = c.d_mats;
     p.nops = nops;
-    // 4-state models: level-parallel kernel (partials, and the logL stage when asked)
-    // auto: the level kernel forms P(t) itself, which saves the P(t) launch (what dominates
-    // small alignments) but repeats the exponentials in every tile (which costs on large ones)
-    const int slots = c.small_waves >= 0 ? c.small_waves : (c.ntiles <= 320 ? 4 : 0);
+    // 4-state models: the traversal of dev_dna.h, or when a level width is asked for, the
+    // level-parallel kernel (partials, and the logL stage when asked)
+    const int slots = c.small_waves;
     const bool small = c.n == 4 && slots > 0 && (nops > 0 || mode == MODE_LOGL);
+    const bool dna = dna_form(c) && (nops > 0 || mode == MODE_LOGL);
     SmallPlan sp;
     if (small) plan_small(c, mode != MODE_PARTIALS, p.br_a, p.br_b, sp);
-    if (small) c.jobs.clear();  // the level-parallel kernel forms P(t) itself
+    bool dna_stage = false;
+    std::vector<int32_t> ranges;
+    if (dna) {
+        // Independent ranges of the list run in workgroups of their own where the tiles alone
+        // leave compute units idle (the branch stage needs both of its partials in one)
+        std::vector<int> newpos;
+        const int max_ranges = mode == MODE_LOGL ? 1 : std::max(1, 16 * c.ncu / c.ntiles);
+        ranges = split_ops(c.nslots, c.pending, max_ranges, newpos);
+        for (PJob &j : c.jobs)
+            if (j.op < nops) j.op = newpos[j.op];
+        p.nbuf = plan_dna(c.nslots, c.pending, ranges, dna_max_buf(c.ntiles, c.ncu));
+        int longest = 0;
+        for (size_t q = 0; q + 1 < ranges.size(); q++) longest = std::max(longest, ranges[q + 1] - ranges[q]);
+        // tip tables of an FP32 range in LDS: their indices, by side
+        int ntab = 0;
+        for (size_t q = 0; f32 && q + 1 < ranges.size(); q++) {
+            int at = 0;
+            for (int i = ranges[q]; i < ranges[q + 1]; i++) {
+                if (c.pending[i].kind <= KIND_TI) c.pending[i].lds_left = at++;
+                if (c.pending[i].kind == KIND_TT) c.pending[i].lds_right = at++;
+            }
+            ntab = std::max(ntab, at);
+        }
+        // A workgroup forms the P(t) data of a short list itself: 1-3 us of its time for 10-60 ops
+        // where the P(t) launch takes 8.  A longer list's data would take the LDS of the buffers
+        // and of further workgroups (512 taxa: 150 KB), and its lanes hold a window of it only.
+        dna_stage = longest <= dna_window(true) - 2 && ntab <= 40;
+        p.small_stage = longest + 1;
+        p.ntip = ntab;
+        p.nlevels = (int)ranges.size() - 1;
+    }
+    if (small || dna_stage) c.jobs.clear();  // these kernels form P(t) themselves
     std::vector<int32_t> perm;
     // (not for the 20-state FP32 traversal, which carries each op's output into the next
     // op of the list's own order)
-    const bool two_orders = !small && !(c.n == 20 && (f32 || p.f64_form == 1)) && alt_order(c, c.pending, perm);
+    const bool two_orders = !small && !dna && !(c.n == 20 && (f32 || p.f64_form == 1)) && alt_order(c, c.pending, perm);
     bool inline_ops = false;
     SmallInline inl;
     p.perm = nullptr;
     const int njobs = (int)c.jobs.size();
-    if (njobs > 0 || small || two_orders) {
+    if (njobs > 0 || small || dna || two_orders) {
         size_t ob = sizeof(DevOp) * nops, jb = sizeof(PJob) * njobs;
-        size_t xb = small ? sizeof(int32_t) * (sp.lvl.size() + sp.tips.size()) : two_orders ? sizeof(int32_t) * nops : 0;
+        size_t xb = small        ? sizeof(int32_t) * (sp.lvl.size() + sp.tips.size())
+                    : dna        ? sizeof(int32_t) * ((ranges.size() + 1) & ~(size_t)1)
+                    : two_orders ? sizeof(int32_t) * nops
+                                 : 0;
         rc = alloc_stage(c, ob + xb + jb);
         if (rc) return rc;
         char *h = (char *)c.h_stage;
@@ -382,13 +509,17 @@ static int run_traversal(Ctx &c, KParams &p, int mode, bool used[3]) {
             p.br_lds_b = sp.br_lds_b;
             p.small_stage = sp.stage ? 1 : 0;
         }
+        if (dna) {
+            std::memcpy(h + ob, ranges.data(), sizeof(int32_t) * ranges.size());
+            p.lvl = (const int32_t *)((char *)c.d_ops + ob);
+        }
         if (two_orders) {
             std::memcpy(h + ob, perm.data(), sizeof(int32_t) * nops);
             p.perm = (const int32_t *)((char *)c.d_ops + ob);
         }
         if (njobs > 0) std::memcpy(h + ob + xb, c.jobs.data(), jb);
         // a short staged list of the level-parallel kernel travels in its kernel arguments
-        inline_ops = small && sp.stage && njobs == 0 && (ob + xb) / 4 <= (size_t)kSmallInlineWords;
+        inline_ops = ((small && sp.stage) || dna_stage) && njobs == 0 && (ob + xb) / 4 <= (size_t)kSmallInlineWords;
         if (inline_ops) {
             inl.nwords = (int32_t)((ob + xb) / 4);
             inl.pad = 0;
@@ -399,15 +530,18 @@ static int run_traversal(Ctx &c, KParams &p, int mode, bool used[3]) {
         if (njobs > 0) {
             HIP_TRY(hipMemcpyAsync(c.d_jobs, h + ob + xb, jb, hipMemcpyHostToDevice, c.stream));
             timing_begin(c, 1);
-            HIP_TRY(f32 ? f32_pmatrix(p, c.d_jobs, njobs, c.stream) : f64_pmatrix(p, c.d_jobs, njobs, c.stream));
+            if (dna) HIP_TRY(dna_pmatrix(p, f32 ? 1 : 0, c.d_jobs, njobs, c.stream));
+            else HIP_TRY(f32 ? f32_pmatrix(p, c.d_jobs, njobs, c.stream) : f64_pmatrix(p, c.d_jobs, njobs, c.stream));
             timing_end(c, 1);
             used[1] = true;
         }
     }
-    if (small) {
+    if (small || dna) {
         const int smode = mode == MODE_LOGL ? MODE_LOGL : MODE_PARTIALS;
+        const SmallInline *in = inline_ops ? &inl : nullptr;
         timing_begin(c, 0);
-        HIP_TRY(small_traverse(p, f32 ? 1 : 0, smode, slots, sp.lds_bytes, inline_ops ? &inl : nullptr, c.stream));
+        if (dna) HIP_TRY(dna_traverse(p, f32 ? 1 : 0, smode, dna_stage, in, c.stream));
+        else HIP_TRY(small_traverse(p, f32 ? 1 : 0, smode, slots, sp.lds_bytes, in, c.stream));
         timing_end(c, 0);
         used[0] = true;
         if (mode == MODE_THETA) {

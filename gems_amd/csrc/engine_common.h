@@ -49,10 +49,10 @@ __host__ __device__ constexpr int mc_leaf(int ncat, int c, int x) {
 // FP32 partial layout inside one (tile, category) block of 64 patterns.  20 states:
 // row groups of 4 states, element (x, p) at ((x / 4) * 64 + p) * 4 + x % 4, so the four
 // matrix-core output rows a lane holds (and the four B-operand rows it feeds) are one
-// 16-byte access; other state counts: element (x, p) at x * 64 + p.
+// 16-byte access; 4 states likewise (one row group); 61 states: element (x, p) at x * 64 + p.
 constexpr bool f32_rg(int n) { return n == 20; }
-__host__ __device__ constexpr int f32_xoff(int n, int x) { return f32_rg(n) ? (x >> 2) * 256 + (x & 3) : x * 64; }
-__host__ __device__ constexpr int f32_loff(int n, int p) { return f32_rg(n) ? p * 4 : p; }
+__host__ __device__ constexpr int f32_xoff(int n, int x) { return n <= 20 ? (x >> 2) * 256 + (x & 3) : x * 64; }
+__host__ __device__ constexpr int f32_loff(int n, int p) { return n <= 20 ? p * 4 : p; }
 // A-fragment k-order of the 20-state form: k-step ks < 4 of lane group g reads state
 // 4g + ks (row group g, element ks), k-step 4 reads state 16 + g (row group 4)
 __host__ __device__ constexpr int f32_kstate(int n, int ks, int g) {
@@ -67,6 +67,17 @@ __host__ __device__ constexpr int f32_orow(int n, int xb, int i) {
     return f32_rg(n) ? (xb == 0 ? i : ((i & 3) == 0 ? 16 + (i >> 2) : -1)) : (xb * 16 + i < n ? xb * 16 + i : -1);
 }
 
+// 4-state traversal (dev_dna.h): P(t) data of one side of an op per group of four categories, in
+// reals: FP64 (form 0) 16 exponentials, FP32 (form 1) four 4 x 4 matrices, and for a tip a
+// table of 19 states x 4 categories x 4 rows
+constexpr int kDnaStates = 19;
+// ops whose tip states a workgroup holds at a time (128 bytes each); a staged list fits with the
+// two that are read ahead
+constexpr int dna_window(bool stage) { return stage ? 64 : 32; }
+constexpr int dna_p_len(int form) { return form == 0 ? 16 : 64; }
+constexpr int dna_table_len() { return kDnaStates * 16; }
+constexpr int dna_side_len(int form, int groups) { return groups * (dna_p_len(form) + (form == 0 ? 0 : dna_table_len())); }
+
 namespace plk {
 
 // Device-side op: one directional partial update.  kind: 0 tip-tip, 1 tip-internal
@@ -76,8 +87,9 @@ struct DevOp {
     int32_t kind;
     int32_t left;   // taxon (kind 0/1) or slot (kind 2)
     int32_t right;  // taxon (kind 0) or slot (kind 1/2)
-    // level-parallel 4-state kernel: LDS buffer of the output / of an internal child
-    // (-1: HBM only), or for a tip child its index among the tips staged in LDS
+    // 4-state kernels: LDS buffer of the output / of an internal child (-1: HBM only); for a
+    // tip child its index among the tips (level-parallel kernel) or the tip tables
+    // (dev_dna.h) staged in LDS
     int32_t lds_out;
     int32_t lds_left;
     int32_t lds_right;
@@ -139,7 +151,8 @@ struct KParams {
     int ntip;                 // tips whose states are staged in LDS
     const int32_t *tips;      // their taxon ids
     int br_lds_a, br_lds_b;   // LDS buffer (or staged tip index) of the branch's two sides
-    int small_stage;          // level-parallel kernel: op list, level bounds and P(t) exponentials staged in LDS
+    int small_stage;          // level-parallel kernel: op list, level bounds and P(t) exponentials staged in LDS;
+                              // dev_dna.h: ops whose P(t) data a workgroup stages at most
     const double *uinv_frag;  // FP64 matrix-core traversal: U^-1 as A fragments (null: not built)
     int f64_form;             // FP64 20/61 states: 1 matrix-core traversal, 0 vector-ALU kernels
 };
@@ -202,7 +215,7 @@ struct Ctx {
     int f64_form = -1;              // FP64 20/61 states, ncat <= 4: 1 matrix cores, 0 vector ALU,
                                     // -1 by state count (61: matrix cores, 20: vector ALU)
     // 4-state models: ops per level run at once by the level-parallel kernel (0: the
-    // category-split kernels; -1: chosen by size, see plk_set_level_waves)
+    // category-split kernels; -1: the traversal of dev_dna.h)
     int small_waves = -1;
     // many-branch derivative buffers (plk_branch_derivs_multi)
     void *d_mparams = nullptr, *d_mitems = nullptr;
@@ -248,6 +261,24 @@ size_t small_lds_bytes(int form, int ncat, int safe, int su, int nbuf, int ntip)
 // extra dynamic LDS of the level-parallel kernel's staged op list (0 = not staged)
 size_t small_stage_bytes(int ncat, int nops, int nlevels);
 
+// 4-state traversal (kernels_dna.hip).  A launch of MODE_PARTIALS may split the op list into
+// independent ranges (op bounds in KParams::lvl, nlevels ranges).
+hipError_t dna_pmatrix(const KParams &p, int form, const PJob *jobs, int njobs, hipStream_t s);
+hipError_t dna_traverse(const KParams &p, int form, int mode, bool stage, const SmallInline *inl, hipStream_t s);
+// nstage, ntab: ops and (FP32) tip tables a workgroup stages
+size_t dna_lds_bytes(int form, int ncat, int waves, int nbuf, int nstage, int ntab);
+// Order the ops by connected component and cut the list into independent ranges (at most
+// max_ranges); the range bounds.  newpos[i] = op i's new position.
+std::vector<int32_t> split_ops(int nslots, std::vector<DevOp> &ops, int max_ranges, std::vector<int> &newpos);
+// Assign LDS buffers (at most max_buf) to the queued ops' outputs by liveness; the number used.
+int plan_dna(int nslots, std::vector<DevOp> &ops, const std::vector<int32_t> &first, int max_buf);
+// the 4-state traversal of dev_dna.h (default) rather than the level or category-split kernels
+inline bool dna_form(const Ctx &c) { return c.n == 4 && c.small_waves < 0; }
+// LDS buffers per wavefront of a launch of `tiles` tiles: with few tiles the LDS is free and
+// a child in memory costs its latency; a large alignment keeps more workgroups per compute
+// unit instead (FP32: 19.4 KB each, so eight; 512 taxa x 100,000 patterns 1258 us at six, 1058 at eight)
+inline int dna_max_buf(int tiles, int ncu) { return tiles <= 2 * ncu ? 8 : 3; }
+
 // Shared host helpers (engine.cpp).
 KParams make_params(Ctx &c);
 // Write-only scratch of a context: a wave that has no real target for a store (a wave
@@ -264,16 +295,18 @@ int f64_form_of(const Ctx &c);
 // Batched partitions: one work item = one workgroup's patterns of one partition: a 64-pattern
 // tile, or mc_batch_patterns patterns of an FP64 20-state one on the matrix cores.  Items are
 // launched in groups, one kernel each: matrix cores (several categories, one category),
-// 20 states, 4 states.
+// 20 states, 4 states (NORM and FP32; FP64 SAFE), 4 states by the category-split kernel.
 struct BatchItem {
     int32_t part;
     int32_t tile;
 };
-enum : int { BATCH_MC = 0, BATCH_MC1 = 1, BATCH_20 = 2, BATCH_4 = 3, BATCH_GROUPS = 4 };
+enum : int { BATCH_MC = 0, BATCH_MC1 = 1, BATCH_20 = 2, BATCH_DNA = 3, BATCH_DNA_SAFE = 4, BATCH_4 = 5, BATCH_GROUPS = 6 };
 constexpr int mc_batch_patterns(int ncat) { return 4 * mc_unit(ncat > 1 ? 2 : 1, ncat); }
+hipError_t batch_pmatrix_dna(int prec, const KParams *params, const PJob *jobs, int njobs, hipStream_t s);
 hipError_t batch_pmatrix(int prec, const KParams *params, const PJob *jobs, int njobs, hipStream_t s);
+// lds: dynamic LDS of the BATCH_DNA launch
 hipError_t batch_traverse(int prec, int group, const KParams *params, const BatchItem *items, int nitems, int grid,
-                          hipStream_t s);
+                          size_t lds, hipStream_t s);
 hipError_t multi_derivs(int prec, int n, int ncw, const KParams *params, const BatchItem *items, int nitems, hipStream_t s);
 hipError_t multi_newton(int prec, int n, int ncw, const KParams *params, const BatchItem *items, int nitems,
                         NewtonState *states, hipStream_t s);

@@ -4,6 +4,7 @@
 // scale counters and fixed-order reduction, so its result is bit-identical to running
 // it alone.  DNA and protein partitions share the launch (the state count is a
 // per-item branch, uniform within a workgroup).
+#include "dev_dna.h"
 #include "dev_f32.h"
 #include "dev_f64.h"
 #include "dev_f64_cat.h"
@@ -52,6 +53,30 @@ __global__ void __launch_bounds__(256) k_batch_traverse_f64(const KParams *param
         const BatchItem it = load_uniform(items + i);
         const KParams P = load_uniform(params + it.part);
         traverse_f64_body<N, MODE_LOGL>(P, it.tile);
+        __syncthreads();
+    }
+}
+
+// one thread per (job, category, state); batched partitions have at most four categories
+template <int FORM>
+__global__ void __launch_bounds__(256) k_batch_pmatrix_dna(const KParams *params, const PJob *jobs, int njobs) {
+    const int idx = blockIdx.x * 256 + threadIdx.x;
+    if (idx >= njobs * 16) return;
+    const PJob j = jobs[idx >> 4];
+    const KParams &P = params[j.pad];
+    const int c = (idx >> 2) & 3, i = idx & 3;
+    if (c >= P.ncat) return;
+    dna_real<FORM> *M = (dna_real<FORM> *)P.mats + (int64_t)j.op * P.mat_stride + j.side * dna_side_len(FORM, 1);
+    dna_pmat<FORM>(P, c, i, j.len, M, j.leaf ? M + dna_p_len(FORM) : nullptr);
+}
+
+template <int FORM, bool SAFE>
+__global__ void __launch_bounds__(256) k_batch_traverse_dna(const KParams *params, const BatchItem *items, int nitems) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    for (int i = blockIdx.x; i < nitems; i += gridDim.x) {
+        const BatchItem it = load_uniform(items + i);
+        const KParams P = load_uniform(params + it.part);
+        traverse_dna_body<FORM, 1, MODE_LOGL, false, SAFE>(P, it.tile, 0, P.nops, smem);
         __syncthreads();
     }
 }
@@ -155,6 +180,14 @@ hipError_t multi_derivs(int prec, int n, int ncw, const KParams *params, const B
     return hipGetLastError();
 }
 
+hipError_t batch_pmatrix_dna(int prec, const KParams *params, const PJob *jobs, int njobs, hipStream_t s) {
+    if (njobs <= 0) return hipSuccess;
+    const dim3 grid((njobs * 16 + 255) / 256);
+    if (prec == PLK_FP64) hipLaunchKernelGGL(k_batch_pmatrix_dna<0>, grid, dim3(256), 0, s, params, jobs, njobs);
+    else hipLaunchKernelGGL(k_batch_pmatrix_dna<1>, grid, dim3(256), 0, s, params, jobs, njobs);
+    return hipGetLastError();
+}
+
 hipError_t batch_pmatrix(int prec, const KParams *params, const PJob *jobs, int njobs, hipStream_t s) {
     if (njobs <= 0) return hipSuccess;
     if (prec == PLK_FP64) hipLaunchKernelGGL(k_batch_pmatrix_f64, dim3(njobs), dim3(256), 0, s, params, jobs);
@@ -163,13 +196,18 @@ hipError_t batch_pmatrix(int prec, const KParams *params, const PJob *jobs, int 
 }
 
 hipError_t batch_traverse(int prec, int group, const KParams *params, const BatchItem *items, int nitems, int grid,
-                          hipStream_t s) {
+                          size_t lds, hipStream_t s) {
     if (nitems <= 0) return hipSuccess;
     const dim3 g((grid <= 0 || grid > nitems) ? nitems : grid), b(256);
     const bool f32 = prec == PLK_FP32;
     switch (group) {
         case BATCH_MC: hipLaunchKernelGGL(k_batch_traverse_f64_cat<2>, g, b, 0, s, params, items, nitems); break;
         case BATCH_MC1: hipLaunchKernelGGL(k_batch_traverse_f64_cat<1>, g, b, 0, s, params, items, nitems); break;
+        case BATCH_DNA:
+            if (f32) hipLaunchKernelGGL((k_batch_traverse_dna<1, false>), g, b, lds, s, params, items, nitems);
+            else hipLaunchKernelGGL((k_batch_traverse_dna<0, false>), g, b, lds, s, params, items, nitems);
+            break;
+        case BATCH_DNA_SAFE: hipLaunchKernelGGL((k_batch_traverse_dna<0, true>), g, b, lds, s, params, items, nitems); break;
         case BATCH_20:
             if (f32) hipLaunchKernelGGL(k_batch_traverse_f32<20>, g, b, 0, s, params, items, nitems);
             else hipLaunchKernelGGL(k_batch_traverse_f64<20>, g, b, 0, s, params, items, nitems);

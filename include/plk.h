@@ -193,13 +193,14 @@ int plk_get_pattern_scaling(plk_ctx *ctx, double *lh, double *scaling);
 int plk_get_pattern_dlogl(plk_ctx *ctx, double *dlogl);
 int plk_set_f64_form(plk_ctx *ctx, int form);
 
-/* 4-state models: 1..4 = level-parallel kernel: the ops are sorted into dependency
- * levels and a 64-pattern tile runs that many independent ops of a level at once
- * (min(ncat, 4) wavefronts each), keeping partials consumed within the launch in LDS and
- * forming P(t) itself (no P(t) launch); 0 = one wavefront per category walking the ops
- * in order after a P(t) launch; -1 (default) = 4 for alignments of at most 320 tiles of
- * 64 patterns, else 0.  Results do not depend on it (partials and scale counts are
- * bit-identical in both forms). */
+/* 4-state models: -1 (default) = one wavefront per 16 patterns and all categories walks the
+ * op list with its products on the matrix cores; 1..4 = level-parallel kernel: the ops are
+ * sorted into dependency levels and a 64-pattern tile runs that many independent ops of a
+ * level at once (min(ncat, 4) wavefronts each), keeping partials consumed within the launch
+ * in LDS and forming P(t) itself (no P(t) launch); 0 = one wavefront per category walking the
+ * ops in order after a P(t) launch.  Partials and scale counts are bit-identical among 0..4,
+ * and in FP32 among all of them; -1 in FP64 sums in another order (a few units in the last
+ * place). */
 int plk_set_level_waves(plk_ctx *ctx, int slots);
 
 /* Kernel timing with HIP events recorded on the context's stream around every launch
