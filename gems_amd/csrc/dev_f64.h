@@ -4,7 +4,7 @@
 // workgroup owns one tile and its wavefronts split the categories (wave w handles
 // c = w, w + nwaves, ...).  Element (ptn, c, x) of a partial is at
 // ((tile*ncat + c)*n + x)*64 + lane, so every load/store of one (c, x) by a wavefront
-// is one contiguous 512-byte segment (20 states: eight 64-byte ones, see f64_xoff).  All tiles are independent across the whole
+// is one contiguous 512-byte segment (20 states: eight 64-byte ones, 61: sixteen 32-byte ones, see f64_xoff).  All tiles are independent across the whole
 // traversal (the reference's packets walk every node for their pattern slice,
 // tree/phylokernelnew.h:2851-2853), so one launch runs the full post-order op list with
 // no grid-wide barrier; each thread only re-reads values it wrote itself.
@@ -51,7 +51,7 @@ __device__ __forceinline__ void stage61_uinv(const double *__restrict__ uinv, do
     __syncthreads();
 }
 
-// acc[x] = sum_i Ec[i][X0 + x] v[i] over i = 0..60 in ascending order, v[i] = V[i * 64];
+// acc[x] = sum_i Ec[i][X0 + x] v[i] over i = 0..60 in ascending order, v[i] = V[f64_xoff(61, i)];
 // X0 is even, so a row segment starts 16-byte aligned; an odd NX reads one padding value.
 template <int X0, int NX>
 __device__ __forceinline__ void cols61(const double *Ec, const double *__restrict__ V, double (&acc)[NX]) {
@@ -59,14 +59,14 @@ __device__ __forceinline__ void cols61(const double *Ec, const double *__restric
     for (int x = 0; x < NX; x++) acc[x] = 0.0;
     double nxt[8];
 #pragma unroll
-    for (int u = 0; u < 8; u++) nxt[u] = V[u * 64];
+    for (int u = 0; u < 8; u++) nxt[u] = V[f64_xoff(61, u)];
     for (int i0 = 0; i0 < 61; i0 += 8) {
         double cur[8];
 #pragma unroll
         for (int u = 0; u < 8; u++) cur[u] = nxt[u];
         // the next block (indices clamped into the partial; values past 60 are not used)
 #pragma unroll
-        for (int u = 0; u < 8; u++) nxt[u] = V[min(i0 + 8 + u, 60) * 64];
+        for (int u = 0; u < 8; u++) nxt[u] = V[f64_xoff(61, min(i0 + 8 + u, 60))];
 #pragma unroll
         for (int u = 0; u < 8; u++) {
             if (i0 + u >= 61) break;
@@ -99,7 +99,7 @@ __device__ __forceinline__ double rows61(const double *Ui, const double (&t)[61]
 #pragma unroll
         for (int q = 0; q < 4; q++) {
             m = fmax(m, fabs(o[q]));
-            dst[(j0 + q) * 64] = o[q];
+            dst[f64_xoff(61, j0 + q)] = o[q];
         }
     }
     double o = 0.0;
@@ -109,7 +109,7 @@ __device__ __forceinline__ double rows61(const double *Ui, const double (&t)[61]
         o = fma(e.x, t[x], o);
         if (x + 1 < 61) o = fma(e.y, t[x + 1], o);
     }
-    dst[60 * 64] = o;
+    dst[f64_xoff(61, 60)] = o;
     return fmax(m, fabs(o));
 }
 
@@ -178,7 +178,7 @@ __device__ inline void pmatrix_f64_body(const KParams &P, const PJob &j, const i
     __syncthreads();
     // the 20-state matrix-core traversal takes the exponentials alone (and its leaf tables in
     // mc_leaf order); otherwise echild is stored [c][i][x]: a column per i, x contiguous (the
-    // 61-state matrix-core fragments and the column-at-a-time kernels read it that way)
+    // column-at-a-time kernels read it that way)
     const bool frag = n == 20 && P.f64_form == 1;
     if (frag) {
         for (int idx = threadIdx.x; idx < nc * n; idx += blockDim.x) {
@@ -246,8 +246,8 @@ __device__ __forceinline__ void op_partial(const KParams &P, const DevOp &op, co
         double l[N], r[N];
 #pragma unroll
         for (int i = 0; i < N; i++) {
-            l[i] = L[i * 64];
-            r[i] = R[i * 64];
+            l[i] = L[f64_xoff(N, i)];
+            r[i] = R[f64_xoff(N, i)];
         }
         for_states<N>([&](const int x) {
             double a = 0.0, b = 0.0;
@@ -265,7 +265,7 @@ __device__ __forceinline__ void op_partial(const KParams &P, const DevOp &op, co
         const double *__restrict__ tl = tabs + (int64_t)sl * block + c * N;
         double r[N];
 #pragma unroll
-        for (int i = 0; i < N; i++) r[i] = R[i * 64];
+        for (int i = 0; i < N; i++) r[i] = R[f64_xoff(N, i)];
         for_states<N>([&](const int x) {
             double b = 0.0;
 #pragma unroll

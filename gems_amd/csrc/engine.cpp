@@ -78,10 +78,10 @@ int ensure_op_capacity(Ctx &c, int nops) {
     return PLK_OK;
 }
 
-// Measured per traversal: 61 states 3.06 -> 0.64 ms on the matrix cores (at most four
-// categories), 20 states 2.13 -> 1.31 ms (100 taxa x 49,994 patterns).
+// Measured per traversal: 61 states 3.06 -> 0.39 ms on the matrix cores (48 taxa x 4,700
+// patterns), 20 states 2.13 -> 1.31 ms (100 taxa x 49,994 patterns).
 int f64_form_of(const Ctx &c) {
-    if (!c.d_uinv_frag || (c.n == 61 && c.ncat > 4)) return 0;
+    if (!c.d_uinv_frag) return 0;
     return c.f64_form >= 0 ? c.f64_form : 1;
 }
 
@@ -480,9 +480,9 @@ static int run_traversal(Ctx &c, KParams &p, int mode, bool used[3]) {
     }
     if (small || dna_stage) c.jobs.clear();  // these kernels form P(t) themselves
     std::vector<int32_t> perm;
-    // (not for the 20-state FP32 traversal, which carries each op's output into the next
-    // op of the list's own order)
-    const bool two_orders = !small && !dna && !(c.n == 20 && (f32 || p.f64_form == 1)) && alt_order(c, c.pending, perm);
+    // (not for the traversals that carry each op's output into the next op of the list's own
+    // order: 20 states in FP32, the matrix-core forms in FP64)
+    const bool two_orders = !small && !dna && !(f32 ? c.n == 20 : p.f64_form == 1) && alt_order(c, c.pending, perm);
     bool inline_ops = false;
     SmallInline inl;
     p.perm = nullptr;
@@ -901,18 +901,20 @@ extern "C" int plk_set_model(plk_ctx *c, const double *eval, const double *evec,
     std::vector<double> uf;
     if (c->d_uinv_frag) {
         uf.assign(mfma64_uinv_frag_size(n), 0.0);
-        const int ks_n = (n + 3) / 4;
         if (n == 20)
             for (int x = 0; x < n; x++)
                 for (int i = 0; i < n; i++) {
                     uf[mc_frag(x, i)] = inv_evec[x * n + i];
                     uf[400 + mc_frag(x, i)] = evec[x * n + i];
                 }
-        // [rb][ks][lane] = U^-1[16 rb + lane % 16][4 ks + lane / 16], zero outside n x n
-        for (size_t f = 0; f < (n == 20 ? 0 : uf.size()); f++) {
-            const int lane = (int)(f % 64), ks = (int)(f / 64) % ks_n, rb = (int)(f / 64) / ks_n;
-            const int j = 16 * rb + lane % 16, x = 4 * ks + lane / 16;
-            if (j < n && x < n) uf[f] = inv_evec[j * n + x];
+        // 61 states: U, then U^-1, as [R][q][s / 2][lane][s % 2] (dev_f64_codon.h), zero outside n x n
+        for (int f = 0; f < (n == 61 ? 64 * 64 : 0); f++) {
+            const int lane = f / 2 % 64, i = lane & 3, b = (lane >> 2) & 3, k = lane >> 4;
+            const int sh = f / 128 % 2 * 2 + f % 2, q = f / 256 % 4, R = f / 1024;
+            const int x = 16 * R + 4 * ((b + sh) & 3) + i, y = 16 * q + 4 * b + k;
+            if (x >= n || y >= n) continue;
+            uf[f] = evec[x * n + y];
+            uf[64 * 64 + f] = inv_evec[x * n + y];
         }
         HIP_TRY(hipMemcpyAsync(c->d_uinv_frag, uf.data(), sizeof(double) * uf.size(), hipMemcpyHostToDevice, c->stream));
     }

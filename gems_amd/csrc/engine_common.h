@@ -18,16 +18,17 @@ constexpr int f32_ksteps(int n) { return (n + 3) / 4; }
 // FP32 leaf-table row length: the matrix-core forms pad a row to whole 16-row blocks
 // (zeros past n), so a lane's four output rows are one aligned 16-byte load
 constexpr int f32_trow(int n) { return n == 4 ? 4 : f32_xblocks(n) * 16; }
-// FP64 matrix-core traversal, constant matrices as A fragments: 61 states U^-1
-// [16-row block][4-state k step][lane], 20 states U^-1 then U (mc_frag order)
-constexpr int mfma64_uinv_frag_size(int n) { return n == 20 ? 800 : ((n + 15) / 16) * ((n + 3) / 4) * 64; }
+// FP64 matrix-core traversal, constant matrices in the kernels' order: 61 states U, then U^-1
+// (dev_f64_codon.h), 20 states U^-1 then U (mc_frag order)
+constexpr int mfma64_uinv_frag_size(int n) { return n == 20 ? 800 : 2 * 64 * 64; }
 // FP64 partial layout inside one (tile, category) block of 64 patterns.  20 states: groups of
 // 8 patterns, element (x, p) at ((p / 8) * 5 + x % 5) * 32 + (x / 5) * 8 + p % 8, so that the 16
 // lanes of the matrix-core traversal that share a category read or write 256 contiguous
-// bytes per k step; other state counts: element (x, p) at x * 64 + p.
+// bytes per k step; 61 states: groups of 4 patterns, element (x, p) at (p / 4) * 244 + x * 4 +
+// p % 4, a wavefront's share in one piece; 4 states: element (x, p) at x * 64 + p.
 constexpr bool f64_rg(int n) { return n == 20; }
-__host__ __device__ constexpr int f64_xoff(int n, int x) { return f64_rg(n) ? (x % 5) * 32 + (x / 5) * 8 : x * 64; }
-__host__ __device__ constexpr int f64_loff(int n, int p) { return f64_rg(n) ? (p >> 3) * 160 + (p & 7) : p; }
+__host__ __device__ constexpr int f64_xoff(int n, int x) { return f64_rg(n) ? (x % 5) * 32 + (x / 5) * 8 : n == 61 ? x * 4 : x * 64; }
+__host__ __device__ constexpr int f64_loff(int n, int p) { return f64_rg(n) ? (p >> 3) * 160 + (p & 7) : n == 61 ? (p >> 2) * 244 + (p & 3) : p; }
 // FP64 matrix-core traversal of 20 states (dev_f64_cat.h): patterns of one wavefront, PG per
 // column; state 5 k + ks is k step ks of lane group k, row 5 i + xb is row i of tile row xb
 constexpr int mc_ncb(int ncat) { return ncat >= 3 ? 4 : ncat; }

@@ -1,7 +1,9 @@
 // FP64 kernels for gfx950: thin __global__ wrappers over the bodies in dev_f64.h.
+#include <algorithm>
+
 #include "dev_f64.h"
 #include "dev_f64_cat.h"
-#include "dev_f64_mfma.h"
+#include "dev_f64_codon.h"
 
 namespace plk {
 namespace {
@@ -30,23 +32,32 @@ __global__ void __launch_bounds__(256, 1) k_traverse_f64_lds61(KParams P) {
     traverse_f64_body<61, MODE, false, true>(P, blockIdx.x);
 }
 
-// matrix-core traversal (20, 61 states, ncat <= 4): one workgroup per 16-pattern block,
-// one wavefront per 16-row block of the states
-// CSPLIT (SAFE scaling only): one workgroup per (block, category), four times the
-// wavefronts for the same work
-// Register budget measured on the 48-taxon x 3,962-pattern codon traversal: the
-// per-category launch runs best at four wavefronts per SIMD (128 VGPRs, a few spilled;
-// 0.58 ms against 0.60 at three and 0.62 at two), the all-category (NORM) one at two
-// (0.76 ms against 0.79 at three and 1.00 at four).
-template <int N, bool CSPLIT>
-__global__ void __launch_bounds__(64 * MfmaShape<N>::RB, CSPLIT ? 4 : 2) k_traverse_f64_mfma(KParams P) {
-    if constexpr (CSPLIT) {
-        const int c = blockIdx.x % P.ncat;
-        traverse_f64_mfma_body<N, MODE_PARTIALS, 1>(P, blockIdx.x / P.ncat, c, c + 1);
-    } else {
-        traverse_f64_mfma_body<N, MODE_PARTIALS, 4>(P, blockIdx.x, 0, P.ncat);
+// 61 states on the matrix cores.  The workgroups load the matrices
+// once and take units in turn: SAFE a unit is (16 patterns, category), NORM four patterns with
+// all categories.
+template <bool SAFE>
+__global__ void __launch_bounds__(SAFE ? 256 : 512, 2) k_traverse_f64_codon(KParams P) {
+    __shared__ unsigned s_ok[2][PLK_GPU_MAX_CATS];
+    __shared__ __attribute__((aligned(16))) double s_ui[64 * 64];
+    const int lane = threadIdx.x & 63, w = wave_id(), ncat = P.ncat;
+    double U[4][4][4];
+#pragma unroll
+    for (int i = 0; i < 64; i++) U[i / 16][i % 4][i / 4 % 4] = P.uinv_frag[(i / 2 * 64 + lane) * 2 + i % 2];
+    for (int i = threadIdx.x; i < 64 * 64; i += blockDim.x) s_ui[i] = P.uinv_frag[64 * 64 + i];
+    __syncthreads();
+    const int units = P.ntiles * (SAFE ? 4 * ncat : 16), n = gridDim.x;
+    int turn = 0;
+    for (int u = blockIdx.x; u < units; u += n) {
+        if (SAFE) traverse_f64_codon_body<true>(P, u / ncat, w, u % ncat, U, s_ui, s_ok, turn);
+        else traverse_f64_codon_body<false>(P, u / 4, u % 4, w, U, s_ui, s_ok, turn);
     }
 }
+
+__global__ void __launch_bounds__(256) k_pmatrix_f64_codon(KParams P, const PJob *__restrict__ jobs) {
+    pmatrix_f64_codon_body(P, jobs[blockIdx.x / P.ncat], blockIdx.x % P.ncat);
+}
+
+__global__ void __launch_bounds__(1024) k_branch_f64_codon(KParams P) { branch_f64_codon_body(P, blockIdx.x); }
 
 // 20 states on the matrix cores; WIDE: 5-8 categories (two wavefronts per pattern unit).
 // PG = 2 takes 160 registers (three wavefronts per SIMD), PG = 1 119 (four).
@@ -115,19 +126,17 @@ hipError_t traverse_n(const KParams &p0, int mode, hipStream_t s) {
     }
     if constexpr (N == 61) {
         if (p.f64_form == 1) {
-            // the op list on the matrix cores, then the branch stage alone (no ops) in the
-            // vector kernel
+            // the op list on the matrix cores, then the branch stage alone (theta: no ops, in
+            // the vector kernel)
             if (p.nops > 0) {
-                if (p.safe)
-                    hipLaunchKernelGGL((k_traverse_f64_mfma<N, true>), dim3(p.ntiles * 4 * p.ncat),
-                                       dim3(64 * MfmaShape<N>::RB), 0, s, p);
-                else
-                    hipLaunchKernelGGL((k_traverse_f64_mfma<N, false>), dim3(p.ntiles * 4), dim3(64 * MfmaShape<N>::RB),
-                                       0, s, p);
+                const int units = p.ntiles * (p.safe ? 4 * p.ncat : 16);
+                const dim3 g(std::min(units, 2 * std::max(1, p.ncu)));  // two stay on a compute unit
+                if (p.safe) hipLaunchKernelGGL(k_traverse_f64_codon<true>, g, dim3(256), 0, s, p);
+                else hipLaunchKernelGGL(k_traverse_f64_codon<false>, g, dim3(64 * p.ncat), 0, s, p);
                 if (mode == MODE_PARTIALS) return hipGetLastError();
                 p.nops = 0;
             }
-            if (mode == MODE_LOGL) hipLaunchKernelGGL((k_traverse_f64<N, MODE_LOGL>), grid, block, 0, s, p);
+            if (mode == MODE_LOGL) hipLaunchKernelGGL(k_branch_f64_codon, grid, dim3(1024), 0, s, p);
             else if (mode == MODE_THETA) hipLaunchKernelGGL((k_traverse_f64<N, MODE_THETA>), grid, block, 0, s, p);
             return hipGetLastError();
         }
@@ -175,7 +184,8 @@ hipError_t f64_theta_newton(const KParams &p, NewtonState *st, hipStream_t s) {
 }
 
 hipError_t f64_pmatrix(const KParams &p, const PJob *jobs, int njobs, hipStream_t s) {
-    hipLaunchKernelGGL(k_pmatrix_f64, dim3(njobs * p.ncat), dim3(256), 0, s, p, jobs);
+    if (p.n == 61 && p.f64_form == 1) hipLaunchKernelGGL(k_pmatrix_f64_codon, dim3(njobs * p.ncat), dim3(256), 0, s, p, jobs);
+    else hipLaunchKernelGGL(k_pmatrix_f64, dim3(njobs * p.ncat), dim3(256), 0, s, p, jobs);
     return hipGetLastError();
 }
 

@@ -172,9 +172,9 @@ int plk_get_exponents(plk_ctx *ctx, int slot, int32_t *exponents);
  * parallelism; fewer reuse each matrix fragment over more patterns).  Results do not
  * depend on it. */
 int plk_set_tile_shape(plk_ctx *ctx, int waves_per_category);
-/* FP64 contexts with 20 states, or 61 states and at most four categories: form 1 runs the
- * partial-likelihood ops on the matrix cores (20 states: 4x4x4 tiles, four categories in one
- * wavefront; 61: 16x16x4 tiles, one workgroup per 16 patterns); form 0 the vector-ALU
+/* FP64 contexts with 20 or 61 states: form 1 runs the traversals on the matrix cores (4x4x4
+ * tiles; 20 states: categories of four or eight patterns side by side in a wavefront; 61:
+ * four patterns of one category a wavefront); form 0 the vector-ALU
  * kernels; -1 (default) the faster one measured, the matrix cores for both.  Same results
  * to rounding (the sums run in a different order); scale counts follow the same rule. */
 /* Side outputs of the last plk_branch_loglik (FP64 form), as computeLikelihoodBranch
