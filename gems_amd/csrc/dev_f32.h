@@ -75,6 +75,71 @@ __device__ inline void pmatrix_f32_body(const KParams &P, const PJob &j, int c0 
     }
 }
 
+// The same for 61 states on 4 x 4 x 4 FP64 tiles (v_mfma_f64_4x4x4_4b_f64, which adds its four
+// terms in order: the sums are those of pmatrix_f32_body bit for bit).  Wavefront xb of four
+// takes the rows 16 xb .. + 15.  Lane j + 4 b + 16 i of a tile holds row 4 b + j, column
+// 4 ks + i of P: a tile is an A fragment of the traversal, and the 16 tiles of a row block are
+// the operands of the leaf-table product as they stand.  All sides of 48 taxa: 92 us with a
+// dot product a thread, 45 now.
+__device__ inline void pmatrix_f32_codon_body(const KParams &P, const PJob &job, const int c) {
+    constexpr int N = 61, KS = 16, FR = 4 * KS * 64, TROW = 64, S = 2;  // S: tiles at once
+    const int lane = threadIdx.x & 63, k = lane >> 4, ncat = P.ncat, su = P.su;
+    const int xb = wave_id(), x = xb * 16 + (lane & 15), i = lane & 3;
+    float *M = (float *)P.mats + (int64_t)job.op * P.mat_stride;
+    float *F = M + ((int64_t)job.side * ncat + c) * FR + xb * KS * 64 + lane;
+    __shared__ double ex[64];
+    if (threadIdx.x < 64) ex[lane] = lane < N ? exp(P.eval[min(lane, N - 1)] * (P.rates[c] * job.len)) : 0.0;
+    __syncthreads();
+    double e[KS], p[KS];
+#pragma unroll
+    for (int q = 0; q < KS; q++) {
+        const int y = 4 * q + k;
+        const double u = P.evec[min(x, N - 1) * N + min(y, N - 1)];
+        e[q] = x < N && y < N ? u * ex[y] : 0.0;
+    }
+#pragma unroll
+    for (int k0 = 0; k0 < KS; k0 += S) {
+        double u[S][KS];
+#pragma unroll
+        for (int g = 0; g < S; g++)
+#pragma unroll
+            for (int q = 0; q < KS; q++) {
+                const int r = 4 * q + k, y = 4 * (k0 + g) + i;
+                const double v = P.inv_evec[min(r, N - 1) * N + min(y, N - 1)];
+                u[g][q] = y < N ? v : 0.0;
+            }
+#pragma unroll
+        for (int g = 0; g < S; g++) p[k0 + g] = 0.0;
+#pragma unroll
+        for (int q = 0; q < KS; q++)
+#pragma unroll
+            for (int g = 0; g < S; g++) p[k0 + g] = __builtin_amdgcn_mfma_f64_4x4x4f64(u[g][q], e[q], p[k0 + g], 0, 0, 0);
+#pragma unroll
+        for (int g = 0; g < S; g++) F[(k0 + g) * 64] = (float)p[k0 + g];
+    }
+    if (!job.leaf) return;
+    float *T = M + (int64_t)2 * ncat * FR + (int64_t)job.side * (su + 1) * ncat * TROW + c * TROW;
+    for (int s0 = 0; s0 < su; s0 += 4 * S) {
+        double t[S][KS], d[S];
+#pragma unroll
+        for (int g = 0; g < S; g++) {
+            d[g] = 0.0;
+#pragma unroll
+            for (int q = 0; q < KS; q++) t[g][q] = P.tipvec[min(s0 + 4 * g + i, su - 1) * N + min(4 * q + k, N - 1)];
+        }
+#pragma unroll
+        for (int q = 0; q < KS; q++)
+#pragma unroll
+            for (int g = 0; g < S; g++) d[g] = __builtin_amdgcn_mfma_f64_4x4x4f64(t[g][q], p[q], d[g], 0, 0, 0);
+#pragma unroll
+        for (int g = 0; g < S; g++) {
+            const int s = s0 + 4 * g + k;
+            if (s < su) T[(int64_t)s * ncat * TROW + x] = (float)d[g];
+        }
+    }
+    if (threadIdx.x < TROW) T[(int64_t)su * ncat * TROW + threadIdx.x] = threadIdx.x < N ? 1.0f : 0.0f;
+}
+
 // ---------------------------------------------------------------------------------------
 // Matrix-core traversal (20 and 61 states).  Workgroup = one 64-pattern tile, one
 // wavefront per category.  Lane l of a wave owns pattern column l%16 of each 16-pattern
@@ -89,7 +154,8 @@ __device__ inline void pmatrix_f32_body(const KParams &P, const PJob &j, int c0 
 // covers only pattern block blk of the tile; `unit` / `nunits` index the workgroup's
 // logL partial sum (by default the tile / the tile count).  A launch whose tile count is
 // just above a multiple of the compute-unit count runs its last tiles as such units, so
-// no compute unit carries a whole extra tile.
+// no compute unit carries a whole extra tile; the 61-state form runs short alignments as
+// units only.
 template <int N, int MODE, int WPC = 1>
 __device__ inline void traverse_f32_mfma_body(const KParams &P, const int tile, const int blk = -1, int unit = -1,
                                               int nunits = -1) {
@@ -460,9 +526,18 @@ __device__ inline void traverse_f32_mfma_body(const KParams &P, const int tile, 
         const int e = expo[(int64_t)P.br_b * P.scale_stride + p] + (atip ? 0 : expo[(int64_t)P.br_a * P.scale_stride + p]);
         const double l = log_lh_expo(lh, e, P.invar[p]);
         if (mine) P.ptn_lh[p] = l;
-        r0 = wave_sum(mine ? l * P.freq[p] : 0.0);
+        r0 = mine ? l * P.freq[p] : 0.0;
+        if constexpr (N > 32) {
+            // by 16-pattern block, so that whole tiles and single-block units add up alike
+#pragma unroll
+            for (int off = 8; off > 0; off >>= 1) r0 += __shfl_down(r0, off, 16);
+            if (blk >= 0) r0 = __shfl(r0, blk * 16, 64);
+        } else {
+            r0 = wave_sum(r0);
+        }
     }
-    finish_tiles(P, r0, 0.0, unit, nunits);
+    if constexpr (N > 32) finish_blocks(P, r0, unit, blk < 0 ? 4 : 1);
+    else finish_tiles(P, r0, 0.0, unit, nunits);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -631,6 +706,10 @@ __device__ inline void traverse_f32_pbw_body(const KParams &P, const int tile) {
     const double ws = wave_sum(contrib);
     if (lane == 0) s_wsum[wave_id()] = ws;
     __syncthreads();
+    if constexpr (N > 32) {
+        finish_blocks(P, s_wsum[(threadIdx.x >> 4) & 3], tile, 4);
+        return;
+    }
     double r0 = 0.0;
     if (threadIdx.x == 0)
         for (int w = 0; w < nwaves() && w < 16; w++) r0 += s_wsum[w];

@@ -30,6 +30,11 @@ __global__ void __launch_bounds__(mfma_threads<WIDE>(), (mfma_min_waves<N, WIDE>
     traverse_f32_mfma_body<N, MODE, WPC>(P, blockIdx.x);
 }
 
+// 61 states
+__global__ void __launch_bounds__(256) k_pmatrix_f32_codon(KParams P, const PJob *__restrict__ jobs) {
+    pmatrix_f32_codon_body(P, jobs[blockIdx.x / P.ncat], blockIdx.x % P.ncat);
+}
+
 // Whole tiles for blockIdx < P.split_full, then single 16-pattern blocks of the remaining
 // tiles (four units per tile), all with one wave per category.
 template <int N, int MODE>
@@ -41,6 +46,12 @@ __global__ void __launch_bounds__(256, 4) k_traverse_f32_mfma_split(KParams P) {
         const int u = b - full;
         traverse_f32_mfma_body<N, MODE, 4>(P, full + u / 4, u % 4, b, gridDim.x);
     }
+}
+
+// 61 states: every tile as four single-block units (rule in traverse_f32_n)
+template <int MODE, bool WIDE>
+__global__ void __launch_bounds__(WIDE ? 512 : 256, 2) k_traverse_f32_units(KParams P) {
+    traverse_f32_mfma_body<61, MODE, 4>(P, blockIdx.x >> 2, blockIdx.x & 3, blockIdx.x, gridDim.x);
 }
 
 template <int N, int MODE>
@@ -78,6 +89,22 @@ hipError_t traverse_f32_n(const KParams &p, int mode, hipStream_t s) {
         if (N > 32) {
             // 61 states: one wave per category (a second one would not fit beside it)
             dim3 block(64 * p.ncat);
+            // Tiles as four units of 16 patterns while all units are resident at once (two
+            // workgroups of four wavefronts a compute unit): a unit reads the fragments that a
+            // tile's four blocks share, but four times the compute units work.  48 taxa, 4
+            // categories: 32 tiles 521 -> 264 us a call, 74 509 -> 317; 176 tiles (704 units,
+            // 512 resident) 555 -> 612.
+            if (4 * p.ntiles <= (p.ncat <= 4 ? 2 : 1) * p.ncu) {
+                const dim3 g4(4 * p.ntiles);
+                if (p.ncat <= 4) {
+                    if (mode == MODE_PARTIALS) hipLaunchKernelGGL((k_traverse_f32_units<MODE_PARTIALS, false>), g4, block, 0, s, p);
+                    else hipLaunchKernelGGL((k_traverse_f32_units<MODE_LOGL, false>), g4, block, 0, s, p);
+                } else {
+                    if (mode == MODE_PARTIALS) hipLaunchKernelGGL((k_traverse_f32_units<MODE_PARTIALS, true>), g4, block, 0, s, p);
+                    else hipLaunchKernelGGL((k_traverse_f32_units<MODE_LOGL, true>), g4, block, 0, s, p);
+                }
+                return hipGetLastError();
+            }
             if (p.ncat <= 4) {
                 if (mode == MODE_PARTIALS) hipLaunchKernelGGL((k_traverse_f32_mfma<N, MODE_PARTIALS, 0, 1>), grid, block, 0, s, p);
                 else hipLaunchKernelGGL((k_traverse_f32_mfma<N, MODE_LOGL, 0, 1>), grid, block, 0, s, p);
@@ -135,7 +162,7 @@ hipError_t f32_pmatrix(const KParams &p, const PJob *jobs, int njobs, hipStream_
             hipLaunchKernelGGL(k_pmatrix_f32<20>, dim3(njobs * p.ncat * f32_xblocks(20)), dim3(256), 0, s, p, jobs);
             break;
         case 61:
-            hipLaunchKernelGGL(k_pmatrix_f32<61>, dim3(njobs * p.ncat * f32_xblocks(61)), dim3(256), 0, s, p, jobs);
+            hipLaunchKernelGGL(k_pmatrix_f32_codon, dim3(njobs * p.ncat), dim3(256), 0, s, p, jobs);
             break;
         default: return hipErrorInvalidValue;
     }

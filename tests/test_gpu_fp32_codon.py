@@ -1,0 +1,25 @@
+"""FP32 61 states: a tile run as four 16-pattern units (while all are resident: up to 128 tiles with 4
+categories, 64 with more, on 256 compute units; the last two sizes lie beyond) against the
+pattern-block shape (up to 4 categories: equal to the bit) and the oracle (1e-6)."""
+import numpy as np
+import pytest
+
+import gems_amd as G
+import support as S
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("ncat,nptn", [(1, 17), (4, 1), (4, 300), (6, 40), (4, 8300), (6, 4200)])
+def test_units_match_whole_tiles(ncat, nptn):
+    p = S.make_problem(61, 6, nptn, np.random.default_rng(ncat + nptn), ncat=ncat, mean_len=0.4, ambiguous=0.05,
+                       compress=False)
+    print("61 states fp32", ncat, nptn, flush=True)
+    g = G.Tree(p, precision=G.FP32)
+    v = g.full_traversal()
+    want = S.Oracle(p, nthreads=8).loglik(0, int(p.nei[0, 0]))
+    assert abs(v - want) <= 1e-6 * abs(want)
+    if ncat <= 4:
+        g.set_tile_shape(0)
+        assert g.full_traversal() == v
+    g.close()
