@@ -73,6 +73,20 @@ __device__ __forceinline__ DevOp load_op(const DevOp *ops, int k) {
     return o;
 }
 
+// Copy a wave-uniform struct out of device memory through the constant address space
+// (scalar loads).
+template <typename T>
+__device__ __forceinline__ T load_uniform(const T *p) {
+    static_assert(sizeof(T) % 8 == 0, "8-byte granular structs only");
+    typedef const __attribute__((address_space(4))) uint64_t *cu64;
+    T v;
+    uint64_t *dst = reinterpret_cast<uint64_t *>(&v);
+    const cu64 src = (cu64)p;
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(T) / 8); i++) dst[i] = src[i];
+    return v;
+}
+
 // Op index of step k for a tile: tiles alternate between the op list's own order and the
 // second order in P.perm (when given), by tile parity flipped every 256 tiles, so that both
 // orders run on every XCD and on most compute units.
@@ -103,10 +117,30 @@ __device__ __forceinline__ int tip_state(const KParams &P, const uint32_t *s, in
 __device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
 __device__ __forceinline__ int nwaves() { return blockDim.x >> 6; }
 
-// Deterministic wavefront sum (fixed shuffle tree); result valid in lane 0.
+// Lane l + OFF's value in lane l, as far as a sum down to lane 0 needs it (OFF = 32: lanes below
+// 32, 16: lanes 0-15, below that within a row of 16): a register operation where a shuffle is an
+// LDS round trip of some 100 cycles.
+template <int OFF>
+__device__ __forceinline__ unsigned lane_down(unsigned v) {
+    if constexpr (OFF == 32) return __builtin_amdgcn_permlane32_swap(v, v, false, false)[1];
+    else if constexpr (OFF == 16) return __builtin_amdgcn_permlane16_swap(v, v, false, false)[1];
+    else return __builtin_amdgcn_update_dpp(0, v, 0x100 | OFF, 0xf, 0xf, true);  // row_shl
+}
+template <int OFF>
+__device__ __forceinline__ double lane_down(double v) {
+    const uint64_t x = __double_as_longlong(v);
+    const uint64_t lo = lane_down<OFF>((unsigned)x), hi = lane_down<OFF>((unsigned)(x >> 32));
+    return __longlong_as_double(lo | hi << 32);
+}
+
+// Deterministic wavefront sum (fixed tree: lanes 32, 16, 8, 4, 2, 1 apart); result valid in lane 0.
 __device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+    v += lane_down<32>(v);
+    v += lane_down<16>(v);
+    v += lane_down<8>(v);
+    v += lane_down<4>(v);
+    v += lane_down<2>(v);
+    v += lane_down<1>(v);
     return v;
 }
 

@@ -607,6 +607,18 @@ extern "C" int plk_device_units(void) {
     return n;
 }
 
+// Two areas of `len` doubles each, all empty (contents are not kept when they grow).
+static hipError_t grow_hand(Ctx &c, HandAreas &a, size_t len) {
+    const size_t need = 2 * (size_t)round_up(sizeof(double) * len, 256);  // areas share no cache line
+    if (need <= a.cap) return hipSuccess;
+    if (a.base) (void)hipFreeAsync(a.base, c.stream);
+    a = HandAreas{};
+    hipError_t e = hipMallocAsync((void **)&a.base, need, c.stream);
+    if (e != hipSuccess) return e;
+    a.cap = need;
+    return hipMemsetAsync(a.base, 0xff, need, c.stream);
+}
+
 extern "C" int64_t plk_memory_required(int nstates, int ncat, int ntaxa, int nptn, int nslots, int precision,
                                        int scaling) {
     int64_t pad = round_up(nptn, 64), block = (int64_t)nstates * ncat, rs = precision == PLK_FP64 ? 8 : 4;
@@ -616,7 +628,7 @@ extern "C" int64_t plk_memory_required(int nstates, int ncat, int ntaxa, int npt
     int64_t theta = pad * block * 8;
     int64_t states = (int64_t)ntaxa * pad;
     int64_t mats = (int64_t)(ntaxa + 1) * mat_stride_of(nstates, ncat, (int)su, precision) * rs;
-    int64_t misc = pad * 8 * 4 + (pad / 64 + 1) * 16;
+    int64_t misc = pad * 8 * 4 + (pad / 64 + 1) * (16 + 144);
     return part + scale + theta + states + mats + misc;
 }
 
@@ -691,6 +703,7 @@ extern "C" int plk_create(plk_ctx **out, int nstates, int ncat, int ntaxa, int n
     CREATE_TRY(hipMallocAsync((void **)&c->d_result, sizeof(double) * 2, c->stream));
     CREATE_TRY(hipMallocAsync((void **)&c->d_counter, sizeof(unsigned), c->stream));
     CREATE_TRY(hipMallocAsync((void **)&c->d_sink, kSinkBytes, c->stream));
+    CREATE_TRY(grow_hand(*c, c->hand, newton_hand_len(c->ntiles)));
     CREATE_TRY(hipMallocAsync((void **)&c->d_newton, sizeof(NewtonState), c->stream));
     c->cap_side = sizeof(double) * (size_t)c->nptn_pad * (ncat + 2);
     CREATE_TRY(hipMallocAsync((void **)&c->d_side, c->cap_side, c->stream));
@@ -716,7 +729,8 @@ extern "C" int plk_create(plk_ctx **out, int nstates, int ncat, int ntaxa, int n
         CREATE_TRY(hipMallocAsync((void **)&c->d_uinv_frag, sizeof(double) * mfma64_uinv_frag_size(n), c->stream));
     CREATE_TRY(hipHostMalloc((void **)&c->h_result, sizeof(double) * 2, hipHostMallocMapped | hipHostMallocCoherent));
     CREATE_TRY(hipHostGetDevicePointer((void **)&c->h_result_dev, c->h_result, 0));
-    CREATE_TRY(hipHostMalloc((void **)&c->h_newton, sizeof(NewtonState), hipHostMallocDefault));
+    CREATE_TRY(hipHostMalloc((void **)&c->h_newton, sizeof(NewtonState), hipHostMallocMapped | hipHostMallocCoherent));
+    CREATE_TRY(hipHostGetDevicePointer((void **)&c->h_newton_dev, c->h_newton, 0));
     for (int i = 0; i < 6; i++) CREATE_TRY(hipEventCreate(&c->ev[i]));
     // zero-initialised state: counters, scale counts and partials of unused slots
     CREATE_TRY(hipMemsetAsync(c->d_counter, 0, sizeof(unsigned), c->stream));
@@ -737,7 +751,8 @@ extern "C" int plk_destroy(plk_ctx *c) {
     void *bufs[] = {c->d_part, c->d_scale, c->d_states, c->d_freq, c->d_invar, c->d_mats, c->d_model,
                     c->d_ops, c->d_jobs, c->d_theta, c->d_buf_scale, c->d_ptn_lh, c->d_tile_sums,
                     c->d_result, c->d_counter, c->d_mparams, c->d_mitems, c->d_mtile, c->d_mres,
-                    c->d_mcount, c->d_newton, c->d_mnewton, c->d_sink, c->d_uinv_frag, c->d_side};
+                    c->d_mcount, c->d_newton, c->d_mnewton, c->d_sink, c->d_uinv_frag, c->d_side,
+                    c->hand.base, c->mhand.base};
     for (void *b : bufs)
         if (b) (void)hipFreeAsync(b, c->stream);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
@@ -785,6 +800,7 @@ extern "C" int plk_reshape(plk_ctx *c, int ntaxa, int nptn, int nslots) {
     }
     if (!rc) rc = grow(*c, (void **)&c->d_theta, c->cap_theta, sizeof(double) * slot);
     if (!rc) rc = grow(*c, (void **)&c->d_tile_sums, c->cap_tiles, sizeof(double) * 2 * 4 * ntiles);
+    if (!rc) HIP_TRY(grow_hand(*c, c->hand, newton_hand_len(ntiles)));
     if (!rc) rc = grow(*c, (void **)&c->d_side, c->cap_side, sizeof(double) * (size_t)pad * (c->ncat + 2));
     if (rc) return rc;
     if (ntiles != c->ntiles && c->mcap) {
@@ -1102,6 +1118,16 @@ extern "C" int plk_loglik_from_theta(plk_ctx *c, double t, double *logl) {
     return PLK_OK;
 }
 
+static int newton_result(const NewtonState &h, double *out, int *evals) {
+    if (evals) *evals = h.evals;
+    switch (h.status) {
+        case NEWTON_OK: *out = h.out; return PLK_OK;
+        case NEWTON_UNDERFLOW: return fail(PLK_ERR_NUMERIC, "Numerical underflow (lh-derivative): use SAFE scaling");
+        case NEWTON_NONFINITE: return fail(PLK_ERR_NUMERIC, "Wrong computeFuncDerv");
+        default: return fail(PLK_ERR_NUMERIC, "Maximum number of iterations exceeded in minimizeNewton");
+    }
+}
+
 extern "C" int plk_newton_branch(plk_ctx *c, int a, int b, double x1, double xguess, double x2, double xacc,
                                  int max_nr, double *out, int *evals) {
     clear_error();
@@ -1120,12 +1146,36 @@ extern "C" int plk_newton_branch(plk_ctx *c, int a, int b, double x1, double xgu
     h.rts = std::min(std::max(xguess, x1), x2);
     h.max_nr = max_nr;
     h.safe = c->safe;
-    HIP_TRY(hipMemcpyAsync(c->d_newton, &h, sizeof(NewtonState), hipMemcpyHostToDevice, c->stream));
     KParams p = make_params(*c);
     p.br_a = a;
     p.br_b = b;
     p.br_len = h.rts;
     bool used[3] = {false, false, false};
+    if (newton_solve_fits(c->n, c->ncat, c->ntiles, c->ncu)) {
+        // The whole solve in one launch, which in the FP64 form also builds theta.  A branch of an
+        // optimisation round (its op, the solve, the host), before and after: DNA 954 patterns 70.5 ->
+        // 33.2 us, 4,783 68.6 -> 34.2, 28,686 90 -> 47; protein 1,941 87 -> 46, 9,027 94 ->
+        // 55; codon 4,015 174 -> 84.
+        const bool f32 = c->prec == PLK_FP32;
+        if (f32 || !c->pending.empty()) {
+            rc = run_traversal(*c, p, f32 ? MODE_THETA : MODE_PARTIALS, used);
+            if (rc) return rc;
+        }
+        const bool timed = !used[2];
+        if (timed) timing_begin(*c, 2);
+        HIP_TRY(newton_solve(p, f32, h, c->hand.next(newton_hand_len(c->ntiles)), c->h_newton_dev, c->stream));
+        if (timed) timing_end(*c, 2);
+        used[2] = true;
+        HIP_TRY(hipStreamSynchronize(c->stream));
+        c->theta_valid = true;
+        c->theta_a = a;
+        c->theta_b = b;
+        if (h.done) {
+            timing_collect(*c, used);
+            return newton_result(h, out, evals);
+        }
+    }
+    HIP_TRY(hipMemcpyAsync(c->d_newton, &h, sizeof(NewtonState), hipMemcpyHostToDevice, c->stream));
     // evaluation 0 builds theta (computeFuncDerv's first call never reuses it)
     rc = run_traversal(*c, p, MODE_THETA, used);
     if (rc) return rc;
@@ -1147,13 +1197,7 @@ extern "C" int plk_newton_branch(plk_ctx *c, int a, int b, double x1, double xgu
         round = std::min(2 * round, 48);
     }
     timing_collect(*c, used);
-    if (evals) *evals = h.evals;
-    switch (h.status) {
-        case NEWTON_OK: *out = h.out; return PLK_OK;
-        case NEWTON_UNDERFLOW: return fail(PLK_ERR_NUMERIC, "Numerical underflow (lh-derivative): use SAFE scaling");
-        case NEWTON_NONFINITE: return fail(PLK_ERR_NUMERIC, "Wrong computeFuncDerv");
-        default: return fail(PLK_ERR_NUMERIC, "Maximum number of iterations exceeded in minimizeNewton");
-    }
+    return newton_result(h, out, evals);
 }
 
 // Buffers of the many-branch launches: per-branch parameters, (branch, tile) items,
@@ -1176,8 +1220,10 @@ static int ensure_multi(Ctx &c, int nbr) {
     HIP_TRY(hipMallocAsync((void **)&c.d_mres, sizeof(double) * 3 * cap, c.stream));
     HIP_TRY(hipMallocAsync((void **)&c.d_mcount, sizeof(unsigned) * cap, c.stream));
     HIP_TRY(hipMallocAsync((void **)&c.d_mnewton, sizeof(NewtonState) * cap, c.stream));
-    HIP_TRY(hipHostMalloc((void **)&c.h_mnewton, sizeof(NewtonState) * cap, hipHostMallocDefault));
+    HIP_TRY(hipHostMalloc((void **)&c.h_mnewton, sizeof(NewtonState) * cap, hipHostMallocMapped | hipHostMallocCoherent));
+    HIP_TRY(hipHostGetDevicePointer((void **)&c.h_mnewton_dev, c.h_mnewton, 0));
     HIP_TRY(hipMemsetAsync(c.d_mcount, 0, sizeof(unsigned) * cap, c.stream));
+    HIP_TRY(grow_hand(c, c.mhand, newton_hand_len(c.ntiles) * cap));
     std::vector<BatchItem> items((size_t)cap * c.ntiles);
     for (int i = 0; i < cap; i++)
         for (int tt = 0; tt < c.ntiles; tt++) items[(size_t)i * c.ntiles + tt] = BatchItem{i, tt};
@@ -1251,7 +1297,18 @@ extern "C" int plk_newton_multi(plk_ctx *c, int nbr, const int *a, const int *b,
             round = std::min(2 * round, 48);
         }
     };
-    rc = run_rounds(eval_only ? 1 : max_nr);
+    const bool whole = c->prec == PLK_FP64 && newton_solve_fits(c->n, c->ncat, c->ntiles, c->ncu);
+    bool finished = false;
+    if (whole) {
+        // every solve in one launch; what did not finish goes on below
+        HIP_TRY(newton_solve_multi(c->n, c->ncat, c->ntiles, (const KParams *)c->d_mparams, c->d_mnewton,
+                                   c->mhand.next(newton_hand_len(c->ntiles) * nbr), c->h_mnewton_dev, nbr, c->stream));
+        HIP_TRY(hipStreamSynchronize(c->stream));
+        finished = true;
+        for (int i = 0; i < nbr && finished; i++) finished = h[i].done != 0;
+        if (!finished) HIP_TRY(hipMemcpyAsync(c->d_mnewton, h, sizeof(NewtonState) * nbr, hipMemcpyHostToDevice, c->stream));
+    }
+    if (!finished) rc = run_rounds(eval_only ? 1 : max_nr);
     if (rc) return rc;
     if (eval_only) {
         for (int i = 0; i < nbr; i++) {

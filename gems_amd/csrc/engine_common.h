@@ -172,6 +172,27 @@ struct NewtonState {
 };
 enum : int { NEWTON_OK = 0, NEWTON_UNDERFLOW = 1, NEWTON_NONFINITE = 2, NEWTON_MAXITER = 3 };
 
+// Exchange places of the one-launch Newton solves (dev_newton.h).  A launch finds its area empty, leaves it
+// used and empties the other one, as far as that was used.
+struct HandArea {
+    double *use, *spare;
+    int64_t spare_len;
+};
+struct HandAreas {
+    double *base = nullptr;
+    size_t cap = 0;             // bytes allocated, both areas
+    int64_t used[2] = {0, 0};   // doubles not empty
+    int turn = 0;
+    HandArea next(int64_t len) {
+        turn ^= 1;
+        const int64_t half = (int64_t)(cap / sizeof(double) / 2);
+        const HandArea a{base + turn * half, base + (turn ^ 1) * half, used[turn ^ 1]};
+        used[turn] = len;
+        used[turn ^ 1] = 0;
+        return a;
+    }
+};
+
 // Host-side context (opaque plk_ctx).
 struct Ctx {
     int dev = 0;
@@ -200,6 +221,8 @@ struct Ctx {
     float *d_sink = nullptr;
     int ncu = 0;  // compute units of the device
     NewtonState *d_newton = nullptr, *h_newton = nullptr;  // device state, pinned host mirror
+    NewtonState *h_newton_dev = nullptr;                   // the mirror's device address
+    HandAreas hand, mhand;                                 // exchange places of one-launch solves: one branch, many
     // host staging (pinned)
     void *h_stage = nullptr;
     size_t h_stage_cap = 0;
@@ -221,8 +244,9 @@ struct Ctx {
     // many-branch derivative buffers (plk_branch_derivs_multi)
     void *d_mparams = nullptr, *d_mitems = nullptr;
     double *d_mtile = nullptr, *d_mres = nullptr;  // 3 values per tile / branch
-    unsigned *d_mcount = nullptr;
+    unsigned *d_mcount = nullptr;                            // per branch: tiles done
     NewtonState *d_mnewton = nullptr, *h_mnewton = nullptr;  // many-branch Newton states (pinned mirror)
+    NewtonState *h_mnewton_dev = nullptr;
     int mcap = 0;
     // allocated sizes (bytes) of the pattern-sized buffers, for plk_reshape
     size_t cap_part = 0, cap_scale = 0, cap_states = 0, cap_pad = 0, cap_theta = 0, cap_tiles = 0;
@@ -245,6 +269,16 @@ hipError_t f64_traverse(const KParams &p, int mode, hipStream_t s);
 hipError_t f64_theta_eval(const KParams &p, int deriv, hipStream_t s);
 hipError_t newton_first(NewtonState *st, const double *result, hipStream_t s);
 hipError_t f64_theta_newton(const KParams &p, NewtonState *st, hipStream_t s);
+// A whole solve per launch (dev_newton.h), while one branch's workgroups take at most a quarter of the
+// wavefront slots (four hardware queues can hold such launches side by side).
+bool newton_solve_fits(int n, int ncat, int ntiles, int ncu);
+// A finished state goes to *out (mapped host memory), an unfinished one (out->done unchanged) is left
+// to the per-evaluation launches.  hand: newton_hand_len doubles per branch, of all-ones bytes.
+constexpr size_t newton_hand_len(int ntiles) { return (size_t)9 * ntiles; }
+hipError_t newton_solve(const KParams &p, bool from_theta, const NewtonState &start, HandArea hand, NewtonState *out,
+                        hipStream_t s);
+hipError_t newton_solve_multi(int n, int ncat, int ntiles, const KParams *params, const NewtonState *start,
+                              HandArea hand, NewtonState *states, int nbr, hipStream_t s);
 hipError_t f32_pmatrix(const KParams &p, const PJob *jobs, int njobs, hipStream_t s);
 hipError_t f32_traverse(const KParams &p, int mode, hipStream_t s);
 hipError_t f32_theta(const KParams &p, hipStream_t s);

@@ -13,20 +13,6 @@ namespace plk {
 namespace {
 using namespace dev;
 
-// Copy a wave-uniform struct out of device memory through the constant address space
-// (scalar loads).
-template <typename T>
-__device__ __forceinline__ T load_uniform(const T *p) {
-    static_assert(sizeof(T) % 8 == 0, "8-byte granular structs only");
-    typedef const __attribute__((address_space(4))) uint64_t *cu64;
-    T v;
-    uint64_t *dst = reinterpret_cast<uint64_t *>(&v);
-    const cu64 src = (cu64)p;
-#pragma unroll
-    for (int i = 0; i < (int)(sizeof(T) / 8); i++) dst[i] = src[i];
-    return v;
-}
-
 __global__ void __launch_bounds__(256) k_batch_pmatrix_f64(const KParams *params, const PJob *jobs) {
     const PJob j = load_uniform(jobs + blockIdx.x);
     const KParams P = load_uniform(params + j.pad);
