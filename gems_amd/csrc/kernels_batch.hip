@@ -29,18 +29,28 @@ __global__ void __launch_bounds__(256) k_batch_pmatrix_f32(const KParams *params
     }
 }
 
-// Persistent when gridDim < nitems: workgroup g takes items g, g + grid, ... (the host
-// orders items by decreasing cost, so the static stride is a longest-first schedule).
 // One kernel per state count: a kernel with both bodies takes the registers and LDS of the
-// larger one for every item (208 registers and 41 KB where DNA alone needs 57 and 19 KB).
-template <int N>
-__global__ void __launch_bounds__(256) k_batch_traverse_f64(const KParams *params, const BatchItem *items, int nitems) {
+// larger one for every item.  TURNS (gridDim < nitems): workgroup g takes items g, g + grid, ...
+// (the host orders items by decreasing cost, so the static stride is a longest-first schedule).
+// Otherwise a workgroup has one item and no loop, out of which the compiler would hoist the
+// constants of exp and log into registers that stay taken through the op list: FP64 20 states
+// 209 registers against 167, 4 states 175 against 125.
+template <bool TURNS, typename F>
+__device__ __forceinline__ void each_item(const KParams *params, const BatchItem *items, int nitems, F &&f) {
     for (int i = blockIdx.x; i < nitems; i += gridDim.x) {
         const BatchItem it = load_uniform(items + i);
         const KParams P = load_uniform(params + it.part);
-        traverse_f64_body<N, MODE_LOGL>(P, it.tile);
+        f(P, it.tile);
+        if (!TURNS) return;
         __syncthreads();
     }
+}
+
+template <int N, bool TURNS>
+__global__ void __launch_bounds__(256) k_batch_traverse_f64(const KParams *params, const BatchItem *items, int nitems) {
+    each_item<TURNS>(params, items, nitems, [&](const KParams &P, int tile) {
+        traverse_f64_body<N, MODE_LOGL>(P, tile);
+    });
 }
 
 // one thread per (job, category, state); batched partitions have at most four categories
@@ -56,37 +66,28 @@ __global__ void __launch_bounds__(256) k_batch_pmatrix_dna(const KParams *params
     dna_pmat<FORM>(P, c, i, j.len, M, j.leaf ? M + dna_p_len(FORM) : nullptr);
 }
 
-template <int FORM, bool SAFE>
+template <int FORM, bool SAFE, bool TURNS>
 __global__ void __launch_bounds__(256) k_batch_traverse_dna(const KParams *params, const BatchItem *items, int nitems) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    for (int i = blockIdx.x; i < nitems; i += gridDim.x) {
-        const BatchItem it = load_uniform(items + i);
-        const KParams P = load_uniform(params + it.part);
-        traverse_dna_body<FORM, 1, MODE_LOGL, false, SAFE>(P, it.tile, 0, P.nops, smem);
-        __syncthreads();
-    }
+    each_item<TURNS>(params, items, nitems, [&](const KParams &P, int tile) {
+        traverse_dna_body<FORM, 1, MODE_LOGL, false, SAFE>(P, tile, 0, P.nops, smem);
+    });
 }
 
 // the 20-state partitions of the matrix-core form: an item is one workgroup's patterns
-template <int PG>
+template <int PG, bool TURNS>
 __global__ void __launch_bounds__(256, 2) k_batch_traverse_f64_cat(const KParams *params, const BatchItem *items, int nitems) {
-    for (int i = blockIdx.x; i < nitems; i += gridDim.x) {
-        const BatchItem it = load_uniform(items + i);
-        const KParams P = load_uniform(params + it.part);
-        traverse_f64_cat_body<MODE_LOGL, PG>(P, it.tile);
-        __syncthreads();
-    }
+    each_item<TURNS>(params, items, nitems, [&](const KParams &P, int tile) {
+        traverse_f64_cat_body<MODE_LOGL, PG>(P, tile);
+    });
 }
 
-template <int N>
+template <int N, bool TURNS>
 __global__ void __launch_bounds__(256) k_batch_traverse_f32(const KParams *params, const BatchItem *items, int nitems) {
-    for (int i = blockIdx.x; i < nitems; i += gridDim.x) {
-        const BatchItem it = load_uniform(items + i);
-        const KParams P = load_uniform(params + it.part);
-        if constexpr (N == 4) traverse_f32_valu_body<4, MODE_LOGL>(P, it.tile);
-        else traverse_f32_mfma_body<N, MODE_LOGL>(P, it.tile);
-        __syncthreads();
-    }
+    each_item<TURNS>(params, items, nitems, [&](const KParams &P, int tile) {
+        if constexpr (N == 4) traverse_f32_valu_body<4, MODE_LOGL>(P, tile);
+        else traverse_f32_mfma_body<N, MODE_LOGL>(P, tile);
+    });
 }
 
 // df/ddf of many branches of one alignment in one launch: item = (branch, tile); each
@@ -181,27 +182,36 @@ hipError_t batch_pmatrix(int prec, const KParams *params, const PJob *jobs, int 
     return hipGetLastError();
 }
 
+template <bool TURNS>
+static void batch_traverse_t(bool f32, int group, const KParams *params, const BatchItem *items, int nitems, dim3 g,
+                             size_t lds, hipStream_t s) {
+    const dim3 b(256);
+    switch (group) {
+        case BATCH_MC: hipLaunchKernelGGL((k_batch_traverse_f64_cat<2, TURNS>), g, b, 0, s, params, items, nitems); break;
+        case BATCH_MC1: hipLaunchKernelGGL((k_batch_traverse_f64_cat<1, TURNS>), g, b, 0, s, params, items, nitems); break;
+        case BATCH_DNA:
+            if (f32) hipLaunchKernelGGL((k_batch_traverse_dna<1, false, TURNS>), g, b, lds, s, params, items, nitems);
+            else hipLaunchKernelGGL((k_batch_traverse_dna<0, false, TURNS>), g, b, lds, s, params, items, nitems);
+            break;
+        case BATCH_DNA_SAFE:
+            hipLaunchKernelGGL((k_batch_traverse_dna<0, true, TURNS>), g, b, lds, s, params, items, nitems);
+            break;
+        case BATCH_20:
+            if (f32) hipLaunchKernelGGL((k_batch_traverse_f32<20, TURNS>), g, b, 0, s, params, items, nitems);
+            else hipLaunchKernelGGL((k_batch_traverse_f64<20, TURNS>), g, b, 0, s, params, items, nitems);
+            break;
+        default:
+            if (f32) hipLaunchKernelGGL((k_batch_traverse_f32<4, TURNS>), g, b, 0, s, params, items, nitems);
+            else hipLaunchKernelGGL((k_batch_traverse_f64<4, TURNS>), g, b, 0, s, params, items, nitems);
+    }
+}
+
 hipError_t batch_traverse(int prec, int group, const KParams *params, const BatchItem *items, int nitems, int grid,
                           size_t lds, hipStream_t s) {
     if (nitems <= 0) return hipSuccess;
-    const dim3 g((grid <= 0 || grid > nitems) ? nitems : grid), b(256);
     const bool f32 = prec == PLK_FP32;
-    switch (group) {
-        case BATCH_MC: hipLaunchKernelGGL(k_batch_traverse_f64_cat<2>, g, b, 0, s, params, items, nitems); break;
-        case BATCH_MC1: hipLaunchKernelGGL(k_batch_traverse_f64_cat<1>, g, b, 0, s, params, items, nitems); break;
-        case BATCH_DNA:
-            if (f32) hipLaunchKernelGGL((k_batch_traverse_dna<1, false>), g, b, lds, s, params, items, nitems);
-            else hipLaunchKernelGGL((k_batch_traverse_dna<0, false>), g, b, lds, s, params, items, nitems);
-            break;
-        case BATCH_DNA_SAFE: hipLaunchKernelGGL((k_batch_traverse_dna<0, true>), g, b, lds, s, params, items, nitems); break;
-        case BATCH_20:
-            if (f32) hipLaunchKernelGGL(k_batch_traverse_f32<20>, g, b, 0, s, params, items, nitems);
-            else hipLaunchKernelGGL(k_batch_traverse_f64<20>, g, b, 0, s, params, items, nitems);
-            break;
-        default:
-            if (f32) hipLaunchKernelGGL(k_batch_traverse_f32<4>, g, b, 0, s, params, items, nitems);
-            else hipLaunchKernelGGL(k_batch_traverse_f64<4>, g, b, 0, s, params, items, nitems);
-    }
+    if (grid <= 0 || grid >= nitems) batch_traverse_t<false>(f32, group, params, items, nitems, dim3(nitems), lds, s);
+    else batch_traverse_t<true>(f32, group, params, items, nitems, dim3(grid), lds, s);
     return hipGetLastError();
 }
 
