@@ -480,7 +480,11 @@ __device__ __forceinline__ double safe_factor(int d) { return d == 0 ? 1.0 : (d 
 // Returns true in the workgroup that wrote the result.
 // E61: the 61-state ops take op_partial_lds61 (ncat <= 4; the workgroup's LDS then holds
 // the 121 KB matrix buffer).
-template <int N, int MODE, bool L3 = false, bool E61 = false>
+// OPS = false: the branch stage alone, without the LDS and registers of the op loop.  The derivatives of
+// 20 states took 217 registers, two workgroups a compute unit; without the loop and with the sums
+// in order (below) 128, four: 97 branches x 3,855 patterns 159 -> 102 us (only bounded to
+// 128 registers they spilled: 326).
+template <int N, int MODE, bool L3 = false, bool E61 = false, bool OPS = true>
 __device__ inline bool traverse_f64_body(const KParams &P, const int tile) {
     static_assert(!E61 || N == 61, "the LDS matrix path is the 61-state one");
     const int lane = threadIdx.x & 63;
@@ -499,7 +503,7 @@ __device__ inline bool traverse_f64_body(const KParams &P, const int tile) {
     if (MODE != MODE_PARTIALS) fill_val(P, P.br_len, s_val[0], MODE == MODE_THETA ? s_val[1] : nullptr, s_val[2]);
 
     // -------- post-order traversal (computePartialLikelihood for every op)
-    for (int k = 0; k < P.nops; k++) {
+    for (int k = 0; k < (OPS ? P.nops : 0); k++) {
         const int ko = op_index(P, tile, k);
         const DevOp op = load_op(P.ops, ko);
         const double *__restrict__ M = (const double *)P.mats + (int64_t)ko * P.mat_stride;
@@ -634,14 +638,33 @@ __device__ inline bool traverse_f64_body(const KParams &P, const int tile) {
             const double *__restrict__ v2 = s_val[2] + c * N;
             const int64_t toff = ((int64_t)tile * ncat + c) * N * 64 + lane;
             double l0 = 0.0, l1 = 0.0, l2 = 0.0;
+            if constexpr (N <= 20) {
+                // all loads of both partials first, then the sums four states at a time: left alone the
+                // compiler reads all 3 N factors from LDS ahead of the first product, into
+                // 120 registers
+                double th[N];
 #pragma unroll
-            for (int i = 0; i < N; i++) {
-                const double a = atip ? tip[i] : A[off + f64_xoff(N, i)];
-                const double th = a * B[off + f64_xoff(N, i)];
-                if (theta) theta[toff + i * 64] = th;  // null: derivatives only (many branches)
-                l0 = fma(v0[i], th, l0);
-                l1 = fma(v1[i], th, l1);
-                l2 = fma(v2[i], th, l2);
+                for (int i = 0; i < N; i++) th[i] = (atip ? tip[i] : A[off + f64_xoff(N, i)]) * B[off + f64_xoff(N, i)];
+                if (theta)  // null: derivatives only (many branches)
+#pragma unroll
+                    for (int i = 0; i < N; i++) theta[toff + i * 64] = th[i];
+#pragma unroll
+                for (int i = 0; i < N; i++) {
+                    if (i % 4 == 0) __builtin_amdgcn_sched_barrier(0);
+                    l0 = fma(v0[i], th[i], l0);
+                    l1 = fma(v1[i], th[i], l1);
+                    l2 = fma(v2[i], th[i], l2);
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < N; i++) {
+                    const double a = atip ? tip[i] : A[off + f64_xoff(N, i)];
+                    const double th = a * B[off + f64_xoff(N, i)];
+                    if (theta) theta[toff + i * 64] = th;
+                    l0 = fma(v0[i], th, l0);
+                    l1 = fma(v1[i], th, l1);
+                    l2 = fma(v2[i], th, l2);
+                }
             }
             s_cat[0][c][lane] = l0;
             s_cat[1][c][lane] = l1;

@@ -99,7 +99,7 @@ template <int N>
 __global__ void __launch_bounds__(256) k_multi_derivs_f64(const KParams *params, const BatchItem *items) {
     const BatchItem it = load_uniform(items + blockIdx.x);
     const KParams P = load_uniform(params + it.part);
-    traverse_f64_body<N, MODE_THETA>(P, it.tile);
+    traverse_f64_body<N, MODE_THETA, false, false, false>(P, it.tile);
 }
 
 template <int N>
@@ -123,7 +123,7 @@ __global__ void __launch_bounds__(256) k_multi_newton(const KParams *params, con
     P.br_len = st->rts;
     bool last;
     if constexpr (F32) last = theta_f32_body<N, true>(P, it.tile);
-    else last = traverse_f64_body<N, MODE_THETA, true>(P, it.tile);
+    else last = traverse_f64_body<N, MODE_THETA, true, false, false>(P, it.tile);
     if (last && threadIdx.x == 0) newton_record(*st, P.result[0], P.result[1], P.result[2]);
 }
 
