@@ -401,7 +401,7 @@ def main():
             "updates_per_step": upd_per_step,
             "logl_fp32": f32["logl"], "logl_rel_err_fp32_vs_oracle": err32,
             "fp64": {"value": f64["ups"], "ms_per_step": f64["ms_per_step"], "logl": f64["logl"],
-                     "logl_rel_err_vs_oracle": err64, "kernel": "k_traverse_f64<20,MODE_LOGL>",
+                     "logl_rel_err_vs_oracle": err64, "kernel": "k_traverse_f64_cat<MODE_LOGL,2>",
                      "kernel_avg_ms": f64["kernel_avg_ms"], "achieved_GBps": f64["achieved"],
                      "roofline_frac": f64["achieved"] / HBM_PEAK_GBS},
             "fp32_over_fp64": f32["ups"] / f64["ups"],
@@ -421,7 +421,7 @@ def main():
         "logl_rel_err_fp32": err32,
         "roofline_fp64": {
             "bound": "hbm", "achieved": f64["achieved"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
-            "frac": f64["achieved"] / HBM_PEAK_GBS, "kernel": "k_traverse_f64<20,MODE_LOGL>",
+            "frac": f64["achieved"] / HBM_PEAK_GBS, "kernel": "k_traverse_f64_cat<MODE_LOGL,2>",
             "kernel_avg_ms": f64["kernel_avg_ms"], "alg_bytes_per_update": f64["bytes_per_update"],
         },
         "roofline": {

@@ -25,7 +25,7 @@
 // lets one branch take a quarter of the wavefront slots, and the workgroups of a branch are
 // neighbours in dispatch order, so the oldest unfinished branch always gets its slots once
 // earlier work drains.  Should they still not come (kernels of more than four queues that hold
-// each other's slots), a wait ends after kSolveWait and the workgroup leaves; the state stays
+// each other's slots), a wait ends after NewtonState::wait and the workgroup leaves; the state stays
 // unfinished and the host solves with one launch per evaluation.
 #pragma once
 
@@ -36,7 +36,6 @@ namespace dev {
 
 __device__ __forceinline__ double hand_empty() { return __longlong_as_double(-1ll); }
 __device__ __forceinline__ bool is_empty(double v) { return __double_as_longlong(v) == -1ll; }
-constexpr uint64_t kSolveWait = 2000000;  // 20 ms of the 100 MHz clock
 
 // L3: many-branch form (the logL of every evaluation, and one more evaluation at the answer where
 // bisection ended on an older point).  THETA: the products are read from P.theta instead of
@@ -55,6 +54,7 @@ __device__ inline void newton_solve_body(const KParams &P, const int wg, const N
     __shared__ NewtonState s_st;
     __shared__ int s_go;
     if (threadIdx.x == 0) s_st = start;
+    const uint64_t wait = (uint64_t)start.wait;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < spare_len; i += (int64_t)gridDim.x * blockDim.x)
         spare[i] = hand_empty();
     // a last workgroup with fewer tiles takes the alignment's last one again and drops its sums
@@ -196,7 +196,7 @@ __device__ inline void newton_solve_body(const KParams &P, const int wg, const N
                         full = full && !is_empty(x[q]);
                     }
                     if (full) break;
-                    if (wall_clock64() - t0 >= kSolveWait) {
+                    if (wall_clock64() - t0 >= wait) {
                         ok = false;
                         break;
                     }

@@ -1153,6 +1153,7 @@ extern "C" int plk_newton_branch(plk_ctx *c, int a, int b, double x1, double xgu
     h.rts = std::min(std::max(xguess, x1), x2);
     h.max_nr = max_nr;
     h.safe = c->safe;
+    h.wait = c->solve_wait;
     KParams p = make_params(*c);
     p.br_a = a;
     p.br_b = b;
@@ -1279,6 +1280,7 @@ extern "C" int plk_newton_multi(plk_ctx *c, int nbr, const int *a, const int *b,
         h[i].rts = std::min(std::max(xguess[i], x1), x2);
         h[i].max_nr = std::max(max_nr, 0);
         h[i].safe = c->safe;
+        h[i].wait = c->solve_wait;
         h[i].eval_only = eval_only ? 1 : 0;
     }
     rc = alloc_stage(*c, sizeof(KParams) * nbr);
@@ -1472,6 +1474,13 @@ extern "C" int plk_get_pattern_dlogl(plk_ctx *c, double *out) {
 extern "C" int plk_set_f64_form(plk_ctx *c, int form) {
     if (!c || form < -1 || form > 1) return fail(PLK_ERR_ARG, "plk_set_f64_form: form must be -1, 0 or 1");
     c->f64_form = form;
+    return PLK_OK;
+}
+
+extern "C" int plk_set_solve_wait(plk_ctx *c, int microseconds) {
+    clear_error();
+    if (!c || microseconds < 0 || microseconds > 1000000) return fail(PLK_ERR_ARG, "plk_set_solve_wait: bad arguments");
+    c->solve_wait = 100 * microseconds;
     return PLK_OK;
 }
 

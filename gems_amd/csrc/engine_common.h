@@ -168,7 +168,8 @@ struct NewtonState {
     double logl_eval, x_eval, logl0;                // many-branch form: logL at the last evaluated
                                                     // length x_eval, and at evaluation 0
     int32_t max_nr, j, done, status, evals, safe;
-    int32_t eval_only, pad;                         // eval_only: evaluate logL at rts and stop
+    int32_t eval_only, wait;                        // eval_only: evaluate logL at rts and stop; wait: bound
+                                                    // of a wait in a one-launch solve (ticks of 10 ns)
 };
 enum : int { NEWTON_OK = 0, NEWTON_UNDERFLOW = 1, NEWTON_NONFINITE = 2, NEWTON_MAXITER = 3 };
 
@@ -222,6 +223,7 @@ struct Ctx {
     int ncu = 0;  // compute units of the device
     NewtonState *d_newton = nullptr, *h_newton = nullptr;  // device state, pinned host mirror
     NewtonState *h_newton_dev = nullptr;                   // the mirror's device address
+    int solve_wait = 2000000;                              // NewtonState::wait: 20 ms
     HandAreas hand, mhand;                                 // exchange places of one-launch solves: one branch, many
     // host staging (pinned)
     void *h_stage = nullptr;

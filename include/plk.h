@@ -203,6 +203,11 @@ int plk_set_f64_form(plk_ctx *ctx, int form);
  * place). */
 int plk_set_level_waves(plk_ctx *ctx, int slots);
 
+/* How long a workgroup of a one-launch Newton solve waits for the others of its branch (default
+ * 20,000 us, at most 1 s).  A solve whose wait ends goes on with one launch per evaluation and
+ * gives the same result; 0 ends nearly every wait. */
+int plk_set_solve_wait(plk_ctx *ctx, int microseconds);
+
 /* Kernel timing with HIP events recorded on the context's stream around every launch
  * of the partial-traversal kernel.  kind: 0 traversal, 1 P(t), 2 derivative. */
 int plk_set_timing(plk_ctx *ctx, int enable);

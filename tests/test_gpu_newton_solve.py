@@ -45,3 +45,27 @@ def test_many_branches_after_fewer():
     for k in (3, 1, len(refs), 7, len(refs)):
         out, lg, st = g.newton_multi(refs[:k], guess[:k])
         assert np.all(st == 0) and np.array_equal(out, first[:k]) and np.array_equal(lg, logl[:k])
+
+
+def test_ended_waits_give_the_same_solves():
+    """With waits of no length the solves go on with one launch per evaluation; the exchange
+    places are clean for the next solve."""
+    p = S.make_problem(4, 12, 3000, np.random.default_rng(4), mean_len=0.2, compress=False)
+    g, h = G.Tree(p, all_directions=True), G.Tree(p, all_directions=True)
+    br, _, _ = g.all_branch_derivs()
+    h.all_branch_derivs()
+
+    def ref(frm, to):
+        return -(to + 1) if to < p.ntaxa else 3 * (to - p.ntaxa) + [int(x) for x in p.nei[to]].index(frm)
+
+    refs = [(ref(v, u), ref(u, v)) for u, v in br]
+    guess = [g.get_length(u, v) for u, v in br]
+    first, logl, _ = g.newton_multi(refs, guess)
+    assert G.lib().plk_set_solve_wait(h.context(), -1) == -1
+    for wait in (0, 20000, 0):
+        assert G.lib().plk_set_solve_wait(h.context(), wait) == 0
+        out, lg, st = h.newton_multi(refs, guess)
+        assert np.all(st == 0) and np.array_equal(out, first) and np.array_equal(lg, logl)
+    for k, (u, v) in enumerate(br[:6]):
+        assert G.lib().plk_set_solve_wait(h.context(), 20000 * (k % 2)) == 0
+        assert g.optimize_one(u, v) == h.optimize_one(u, v)
