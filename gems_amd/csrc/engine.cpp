@@ -458,23 +458,30 @@ static int run_traversal(Ctx &c, KParams &p, int mode, bool used[3]) {
         ranges = split_ops(c.nslots, c.pending, max_ranges, newpos);
         for (PJob &j : c.jobs)
             if (j.op < nops) j.op = newpos[j.op];
-        p.nbuf = plan_dna(c.nslots, c.pending, ranges, dna_max_buf(c.ntiles, c.ncu));
-        int longest = 0;
-        for (size_t q = 0; q + 1 < ranges.size(); q++) longest = std::max(longest, ranges[q + 1] - ranges[q]);
-        // tip tables of an FP32 range in LDS: their indices, by side
-        int ntab = 0;
+        int longest = 0, ntab = 0;
+        for (size_t q = 0; q + 1 < ranges.size(); q++) {
+            longest = std::max(longest, ranges[q + 1] - ranges[q]);
+            int tabs = 0;  // tip tables of an FP32 range
+            for (int i = ranges[q]; f32 && i < ranges[q + 1]; i++)
+                tabs += (c.pending[i].kind <= KIND_TI) + (c.pending[i].kind == KIND_TT);
+            ntab = std::max(ntab, tabs);
+        }
+        // A workgroup forms the P(t) data of a short list itself: 1-3 us of its time for 10-60 ops
+        // where the P(t) launch takes 8.  A longer list's data would take the LDS of the buffers
+        // and of further workgroups (512 taxa: 150 KB), and its lanes hold a window of it only.
+        // With five to eight categories it is twice the size: only where kDnaMinBuf buffers fit too.
+        dna_stage = longest <= dna_window(true) - 2 && ntab <= 40 &&
+                    dna_buf_room(f32 ? 1 : 0, c.ncat, longest + 1, ntab) >= kDnaMinBuf;
+        const int room = dna_stage ? dna_buf_room(f32 ? 1 : 0, c.ncat, longest + 1, ntab) : dna_buf_room(f32 ? 1 : 0, c.ncat, 0, 0);
+        p.nbuf = plan_dna(c.nslots, c.pending, ranges, std::min(dna_max_buf(c.ntiles, c.ncu), room));
+        // indices of the tip tables in LDS, by side
         for (size_t q = 0; f32 && q + 1 < ranges.size(); q++) {
             int at = 0;
             for (int i = ranges[q]; i < ranges[q + 1]; i++) {
                 if (c.pending[i].kind <= KIND_TI) c.pending[i].lds_left = at++;
                 if (c.pending[i].kind == KIND_TT) c.pending[i].lds_right = at++;
             }
-            ntab = std::max(ntab, at);
         }
-        // A workgroup forms the P(t) data of a short list itself: 1-3 us of its time for 10-60 ops
-        // where the P(t) launch takes 8.  A longer list's data would take the LDS of the buffers
-        // and of further workgroups (512 taxa: 150 KB), and its lanes hold a window of it only.
-        dna_stage = longest <= dna_window(true) - 2 && ntab <= 40;
         p.small_stage = longest + 1;
         p.ntip = ntab;
         p.nlevels = (int)ranges.size() - 1;

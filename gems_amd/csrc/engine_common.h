@@ -304,6 +304,20 @@ hipError_t dna_pmatrix(const KParams &p, int form, const PJob *jobs, int njobs, 
 hipError_t dna_traverse(const KParams &p, int form, int mode, bool stage, const SmallInline *inl, hipStream_t s);
 // nstage, ntab: ops and (FP32) tip tables a workgroup stages
 size_t dna_lds_bytes(int form, int ncat, int waves, int nbuf, int nstage, int ntab);
+// LDS that a launch may ask for: a workgroup's 160 KB less the kernels' own arrays (528 bytes).
+// dna_traverse refuses a launch that is over it.
+constexpr size_t kDnaLdsMax = 160 * 1024 - 1024;
+// buffers per wavefront that fit beside nstage ops and ntab tip tables
+inline int dna_buf_room(int form, int ncat, int nstage, int ntab) {
+    const int waves = ncat >= 3 ? 4 : ncat;
+    const size_t fixed = dna_lds_bytes(form, ncat, waves, 0, nstage, ntab);
+    const size_t per_buf = dna_lds_bytes(form, ncat, waves, 1, 0, 0) - dna_lds_bytes(form, ncat, waves, 0, 0, 0);
+    return fixed < kDnaLdsMax ? (int)((kDnaLdsMax - fixed) / per_buf) : 0;
+}
+// Staging stands back for this many of them (6 categories): FP32 logL of 38 and 40 taxa, one buffer or two
+// beside the staged data 51-55 us, three and the P(t) launch 50-51; FP64 gradients of 8-20 taxa
+// and NNI moves, five buffers beside it 63-111 us and 370-484, without it 70-118 and 419-529.
+constexpr int kDnaMinBuf = 3;
 // Order the ops by connected component and cut the list into independent ranges (at most
 // max_ranges); the range bounds.  newpos[i] = op i's new position.
 std::vector<int32_t> split_ops(int nslots, std::vector<DevOp> &ops, int max_ranges, std::vector<int> &newpos);
@@ -313,7 +327,8 @@ int plan_dna(int nslots, std::vector<DevOp> &ops, const std::vector<int32_t> &fi
 inline bool dna_form(const Ctx &c) { return c.n == 4 && c.small_waves < 0; }
 // LDS buffers per wavefront of a launch of `tiles` tiles: with few tiles the LDS is free and
 // a child in memory costs its latency; a large alignment keeps more workgroups per compute
-// unit instead (FP32: 19.4 KB each, so eight; 512 taxa x 100,000 patterns 1258 us at six, 1058 at eight)
+// unit instead (FP32: 19.4 KB each, so eight; 512 taxa x 100,000 patterns 1258 us at six, 1058 at eight).
+// (At most: dna_buf_room.)
 inline int dna_max_buf(int tiles, int ncu) { return tiles <= 2 * ncu ? 8 : 3; }
 
 // Shared host helpers (engine.cpp).

@@ -209,6 +209,7 @@ static void batch_traverse_t(bool f32, int group, const KParams *params, const B
 hipError_t batch_traverse(int prec, int group, const KParams *params, const BatchItem *items, int nitems, int grid,
                           size_t lds, hipStream_t s) {
     if (nitems <= 0) return hipSuccess;
+    if (lds > kDnaLdsMax) return hipErrorInvalidConfiguration;
     const bool f32 = prec == PLK_FP32;
     if (grid <= 0 || grid >= nitems) batch_traverse_t<false>(f32, group, params, items, nitems, dim3(nitems), lds, s);
     else batch_traverse_t<true>(f32, group, params, items, nitems, dim3(grid), lds, s);

@@ -48,6 +48,7 @@ hipError_t launch(const KParams &p, bool stage, const SmallInline *inl, hipStrea
     const int waves = p.ncat >= 3 ? 4 : p.ncat;
     const dim3 grid(p.ntiles, MODE == MODE_PARTIALS && p.nlevels > 1 ? p.nlevels : 1), block(64 * waves);
     const size_t lds = dna_lds_bytes(FORM, p.ncat, waves, p.nbuf, stage ? p.small_stage : 0, stage ? p.ntip : 0);
+    if (lds > kDnaLdsMax) return hipErrorInvalidConfiguration;
     if (inl) hipLaunchKernelGGL((k_traverse_dna_inl<FORM, CG, MODE, SAFE>), grid, block, lds, s, p, *inl);
     else if (stage) hipLaunchKernelGGL((k_traverse_dna<FORM, CG, MODE, true, SAFE>), grid, block, lds, s, p);
     else hipLaunchKernelGGL((k_traverse_dna<FORM, CG, MODE, false, SAFE>), grid, block, lds, s, p);

@@ -1,0 +1,44 @@
+"""What the host code plans and launches, on the CPU (hip_record.cpp plays the HIP runtime)."""
+import os
+
+import pytest
+
+import recorded as R
+
+LDS = 160 * 1024  # of a workgroup on gfx950
+
+
+@pytest.mark.skipif(not os.path.exists(R.READELF), reason="llvm-readelf not available")
+@pytest.mark.parametrize("ncat", range(1, 9))
+def test_lds_of_every_launch_fits(ncat):
+    """4 states, both forms and scaling modes, short and long alignments and every kind of op list
+    (post-order, all directions, the moves of all branches); no call is refused."""
+    got = R.run(f"""
+    out, ncat = [], {ncat}
+    for taxa in (5, 9, 12, 20, 30, 38, 40, 41, 64, 100, 160):
+        for nptn in (1, 1000, 16000, 64 * 512, 64 * 512 + 1):
+            if nptn > 16000 and taxa not in (20, 41, 100):
+                continue
+            p = S.make_problem(4, taxa, 1, np.random.default_rng(taxa), ncat=ncat, compress=False)
+            p.states, p.freq, p.nptn = np.repeat(p.states, nptn, 1), np.ones(nptn), nptn
+            internal = [(u, int(v)) for u in range(taxa, 2 * taxa - 2) for v in p.nei[u] if v > u]
+            for prec, safe in ((G.FP64, 0), (G.FP64, 1), (G.FP32, 0)):
+                t = G.Tree(p, precision=prec, scaling=safe, all_directions=2 if taxa <= 100 and nptn <= 1000 else 1)
+                rc = [called(t.full_traversal)]
+                G.lib().plk_tree_clear_all(t.h)
+                rc.append(called(t.derivs, 0, int(p.nei[0, 0])))
+                G.lib().plk_tree_clear_all(t.h)
+                rc.append(called(t.all_branch_derivs))
+                if taxa <= 100 and nptn <= 1000 and prec == G.FP64:
+                    G.lib().plk_tree_clear_all(t.h)
+                    rc.append(called(t.nni_evaluate, internal))
+                out.append((taxa, nptn, prec, safe, rc, sorted(set((n, l) for n, l, _ in launches()))))
+                t.close()
+    print(json.dumps(out))
+    """)
+    static = R.static_lds()
+    for taxa, nptn, prec, safe, rc, kernels in got:
+        assert not any(rc), (taxa, nptn, prec, safe, rc)
+        assert any("k_traverse_dna" in name for name, _ in kernels)
+        for name, lds in kernels:
+            assert lds + static[name] <= LDS, (taxa, nptn, prec, safe, name, lds)
