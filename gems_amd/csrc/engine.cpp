@@ -435,6 +435,16 @@ static bool alt_order(const Ctx &c, const std::vector<DevOp> &ops, std::vector<i
 static int run_traversal(Ctx &c, KParams &p, int mode, bool used[3]) {
     const int nops = (int)c.pending.size();
     const bool f32 = c.prec == PLK_FP32;
+    // A call that fails leaves the queue as it found it (the ops perhaps in another order): the
+    // next one forms P(t) of these ops, in whichever kernel it takes.
+    struct Keep {
+        std::vector<PJob> &jobs;
+        const size_t queued = jobs.size();
+        bool failed = true;
+        ~Keep() {
+            if (failed) jobs.resize(queued);
+        }
+    } keep{c.jobs};
     if (f32 && mode == MODE_LOGL) c.jobs.push_back(PJob{nops, 0, 0, 0, p.br_len});
     int rc = ensure_op_capacity(c, nops + 1);
     if (rc) return rc;
@@ -486,7 +496,6 @@ static int run_traversal(Ctx &c, KParams &p, int mode, bool used[3]) {
         p.ntip = ntab;
         p.nlevels = (int)ranges.size() - 1;
     }
-    if (small || dna_stage) c.jobs.clear();  // these kernels form P(t) themselves
     std::vector<int32_t> perm;
     // (not for the traversals that carry each op's output into the next op of the list's own
     // order: 20 states in FP32, the matrix-core forms in FP64)
@@ -494,7 +503,7 @@ static int run_traversal(Ctx &c, KParams &p, int mode, bool used[3]) {
     bool inline_ops = false;
     SmallInline inl;
     p.perm = nullptr;
-    const int njobs = (int)c.jobs.size();
+    const int njobs = small || dna_stage ? 0 : (int)c.jobs.size();  // (these kernels form P(t) themselves)
     if (njobs > 0 || small || dna || two_orders) {
         size_t ob = sizeof(DevOp) * nops, jb = sizeof(PJob) * njobs;
         size_t xb = small        ? sizeof(int32_t) * (sp.lvl.size() + sp.tips.size())
@@ -584,6 +593,7 @@ static int run_traversal(Ctx &c, KParams &p, int mode, bool used[3]) {
     c.updates += (int64_t)nops * c.nptn;
     c.pending.clear();
     c.jobs.clear();
+    keep.failed = false;
     return PLK_OK;
 }
 

@@ -42,3 +42,33 @@ def test_lds_of_every_launch_fits(ncat):
         assert any("k_traverse_dna" in name for name, _ in kernels)
         for name, lds in kernels:
             assert lds + static[name] <= LDS, (taxa, nptn, prec, safe, name, lds)
+
+
+@pytest.mark.parametrize("prec", ["FP64", "FP32"])
+def test_failed_launch_keeps_the_transition_matrices_to_come(prec):
+    """After a refused traversal the next call forms P(t) of all queued ops, whichever kernel it
+    takes, and of its own branch once."""
+    got = R.run(f"""
+    p = S.make_problem(4, 12, 300, np.random.default_rng(1), compress=False)
+    w = int(p.nei[0, 0])
+    out = []
+    for waves in (0, 1, -1):
+        calls = []
+        for fails in (0, 1, 3):
+            t = G.Tree(p, precision=G.{prec})
+            rec.rec_fail(b"k_traverse")
+            rc = [called(t.loglik, 0, w) for _ in range(fails)]
+            rec.rec_fail(b"")
+            t.set_level_waves(waves)
+            launches()
+            rc.append(called(t.loglik, 0, w))
+            calls.append((rc, launches()))
+            t.close()
+        out.append(calls)
+    print(json.dumps(out))
+    """)
+    for fresh, *after in got:
+        assert fresh[0] == [0]
+        for rc, kernels in after:
+            assert all(rc[:-1]) and rc[-1] == 0
+            assert kernels == fresh[1]
