@@ -637,6 +637,20 @@ static hipError_t grow_hand(Ctx &c, HandAreas &a, size_t len) {
     return hipMemsetAsync(a.base, 0xff, need, c.stream);
 }
 
+// A one-launch solve with its exchange places; both areas are filled again after a launch that failed.
+template <typename F>
+static hipError_t with_hand(Ctx &c, HandAreas &a, int64_t len, F &&launch) {
+    if (a.spoilt) {
+        const hipError_t e = hipMemsetAsync(a.base, 0xff, a.cap, c.stream);
+        if (e != hipSuccess) return e;
+        a.used[0] = a.used[1] = 0;
+    }
+    a.spoilt = true;
+    const hipError_t e = launch(a.next(len));
+    a.spoilt = e != hipSuccess;
+    return e;
+}
+
 extern "C" int64_t plk_memory_required(int nstates, int ncat, int ntaxa, int nptn, int nslots, int precision,
                                        int scaling) {
     int64_t pad = round_up(nptn, 64), block = (int64_t)nstates * ncat, rs = precision == PLK_FP64 ? 8 : 4;
@@ -1188,7 +1202,9 @@ extern "C" int plk_newton_branch(plk_ctx *c, int a, int b, double x1, double xgu
         }
         const bool timed = !used[2];
         if (timed) timing_begin(*c, 2);
-        HIP_TRY(newton_solve(p, f32, h, c->hand.next(newton_hand_len(c->ntiles)), c->h_newton_dev, c->stream));
+        HIP_TRY(with_hand(*c, c->hand, newton_hand_len(c->ntiles), [&](const HandArea &hand) {
+            return newton_solve(p, f32, h, hand, c->h_newton_dev, c->stream);
+        }));
         if (timed) timing_end(*c, 2);
         used[2] = true;
         HIP_TRY(hipStreamSynchronize(c->stream));
@@ -1327,8 +1343,10 @@ extern "C" int plk_newton_multi(plk_ctx *c, int nbr, const int *a, const int *b,
     bool finished = false;
     if (whole) {
         // every solve in one launch; what did not finish goes on below
-        HIP_TRY(newton_solve_multi(c->n, c->ncat, c->ntiles, (const KParams *)c->d_mparams, c->d_mnewton,
-                                   c->mhand.next(newton_hand_len(c->ntiles) * nbr), c->h_mnewton_dev, nbr, c->stream));
+        HIP_TRY(with_hand(*c, c->mhand, newton_hand_len(c->ntiles) * nbr, [&](const HandArea &hand) {
+            return newton_solve_multi(c->n, c->ncat, c->ntiles, (const KParams *)c->d_mparams, c->d_mnewton, hand,
+                                      c->h_mnewton_dev, nbr, c->stream);
+        }));
         HIP_TRY(hipStreamSynchronize(c->stream));
         finished = true;
         for (int i = 0; i < nbr && finished; i++) finished = h[i].done != 0;

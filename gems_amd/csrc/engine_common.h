@@ -184,6 +184,7 @@ struct HandAreas {
     size_t cap = 0;             // bytes allocated, both areas
     int64_t used[2] = {0, 0};   // doubles not empty
     int turn = 0;
+    bool spoilt = false;        // a launch failed, so that neither area is what it was to be
     HandArea next(int64_t len) {
         turn ^= 1;
         const int64_t half = (int64_t)(cap / sizeof(double) / 2);

@@ -72,3 +72,24 @@ def test_failed_launch_keeps_the_transition_matrices_to_come(prec):
         for rc, kernels in after:
             assert all(rc[:-1]) and rc[-1] == 0
             assert kernels == fresh[1]
+
+
+def test_exchange_places_after_a_failed_solve():
+    """Every one-launch solve finds its exchange places empty, also after launches that failed."""
+    got = R.run("""
+    p = S.make_problem(4, 12, 300, np.random.default_rng(1), compress=False)
+    t = G.Tree(p, all_directions=2)
+    w, inner = int(p.nei[0, 0]), [(u, int(v)) for u in range(12, 22) for v in p.nei[u] if v > u]
+    out = []
+    for step in ("one", "all", "one", "all", "", "one", "all", "", "one", "one", "all", "all"):
+        rec.rec_fail(b"" if step else b"k_newton_solve")
+        if step != "all":
+            rc = called(t.optimize_one, 0, w)
+        if step != "one":
+            rc = called(t.nni_evaluate, inner)
+        out.append((step, rc, rec.rec_dirty()))
+    print(json.dumps([out, [n for n, _, _ in launches() if "newton_solve" in n]]))
+    """)
+    assert all((rc == 0) == bool(step) for step, rc, _ in got[0])
+    assert any("solve_multi" in n for n in got[1]) and any("solveI" in n for n in got[1])
+    assert not any(dirty for _, _, dirty in got[0]), got[0]
