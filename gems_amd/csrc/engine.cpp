@@ -634,12 +634,17 @@ static hipError_t grow_hand(Ctx &c, HandAreas &a, size_t len) {
     hipError_t e = hipMallocAsync((void **)&a.base, need, c.stream);
     if (e != hipSuccess) return e;
     a.cap = need;
-    return hipMemsetAsync(a.base, 0xff, need, c.stream);
+    e = hipMemsetAsync(a.base, 0xff, need, c.stream);
+    a.spoilt = e != hipSuccess;
+    return e;
 }
 
-// A one-launch solve with its exchange places; both areas are filled again after a launch that failed.
+// A one-launch solve with its exchange places, allocated where they are first needed; both areas are filled
+// again after a launch that failed.
 template <typename F>
 static hipError_t with_hand(Ctx &c, HandAreas &a, int64_t len, F &&launch) {
+    const hipError_t grown = grow_hand(c, a, len);
+    if (grown != hipSuccess) return grown;
     if (a.spoilt) {
         const hipError_t e = hipMemsetAsync(a.base, 0xff, a.cap, c.stream);
         if (e != hipSuccess) return e;
@@ -735,7 +740,7 @@ extern "C" int plk_create(plk_ctx **out, int nstates, int ncat, int ntaxa, int n
     CREATE_TRY(hipMallocAsync((void **)&c->d_result, sizeof(double) * 2, c->stream));
     CREATE_TRY(hipMallocAsync((void **)&c->d_counter, sizeof(unsigned), c->stream));
     CREATE_TRY(hipMallocAsync((void **)&c->d_sink, kSinkBytes, c->stream));
-    CREATE_TRY(grow_hand(*c, c->hand, newton_hand_len(c->ntiles)));
+    if (newton_solve_fits(nstates, ncat, c->ntiles, c->ncu)) CREATE_TRY(grow_hand(*c, c->hand, newton_hand_len(c->ntiles)));
     CREATE_TRY(hipMallocAsync((void **)&c->d_newton, sizeof(NewtonState), c->stream));
     c->cap_side = sizeof(double) * (size_t)c->nptn_pad * (ncat + 2);
     CREATE_TRY(hipMallocAsync((void **)&c->d_side, c->cap_side, c->stream));
@@ -832,15 +837,16 @@ extern "C" int plk_reshape(plk_ctx *c, int ntaxa, int nptn, int nslots) {
     }
     if (!rc) rc = grow(*c, (void **)&c->d_theta, c->cap_theta, sizeof(double) * slot);
     if (!rc) rc = grow(*c, (void **)&c->d_tile_sums, c->cap_tiles, sizeof(double) * 2 * 4 * ntiles);
-    if (!rc) HIP_TRY(grow_hand(*c, c->hand, newton_hand_len(ntiles)));
+    if (!rc && newton_solve_fits(c->n, c->ncat, ntiles, c->ncu)) HIP_TRY(grow_hand(*c, c->hand, newton_hand_len(ntiles)));
     if (!rc) rc = grow(*c, (void **)&c->d_side, c->cap_side, sizeof(double) * (size_t)pad * (c->ncat + 2));
     if (rc) return rc;
     if (ntiles != c->ntiles && c->mcap) {
         // the many-branch buffers hold (branch, tile) items: rebuilt on next use
-        void *old[] = {c->d_mparams, c->d_mitems, c->d_mtile, c->d_mres, c->d_mcount, c->d_mnewton};
+        void *old[] = {c->d_mparams, c->d_mitems, c->d_mtile, c->d_mres, c->d_mcount, c->d_mnewton, c->mhand.base};
         for (void *q : old)
             if (q) (void)hipFreeAsync(q, c->stream);
         if (c->h_mnewton) (void)hipHostFree(c->h_mnewton);
+        c->mhand = HandAreas{};
         c->d_mparams = c->d_mitems = nullptr;
         c->d_mtile = c->d_mres = nullptr;
         c->d_mcount = nullptr;
@@ -1264,7 +1270,6 @@ static int ensure_multi(Ctx &c, int nbr) {
     HIP_TRY(hipHostMalloc((void **)&c.h_mnewton, sizeof(NewtonState) * cap, hipHostMallocMapped | hipHostMallocCoherent));
     HIP_TRY(hipHostGetDevicePointer((void **)&c.h_mnewton_dev, c.h_mnewton, 0));
     HIP_TRY(hipMemsetAsync(c.d_mcount, 0, sizeof(unsigned) * cap, c.stream));
-    HIP_TRY(grow_hand(c, c.mhand, newton_hand_len(c.ntiles) * cap));
     std::vector<BatchItem> items((size_t)cap * c.ntiles);
     for (int i = 0; i < cap; i++)
         for (int tt = 0; tt < c.ntiles; tt++) items[(size_t)i * c.ntiles + tt] = BatchItem{i, tt};

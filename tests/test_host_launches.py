@@ -93,3 +93,30 @@ def test_exchange_places_after_a_failed_solve():
     assert all((rc == 0) == bool(step) for step, rc, _ in got[0])
     assert any("solve_multi" in n for n in got[1]) and any("solveI" in n for n in got[1])
     assert not any(dirty for _, _, dirty in got[0]), got[0]
+
+
+def test_exchange_places_are_allocated_for_solves_only():
+    """Derivatives of all branches allocate none (8 + 24 bytes a branch and tile is what they need), nor
+    do sizes that the one-launch solve does not take; all is given back."""
+    got = R.run("""
+    out = []
+    for nptn in (6400, 64 * 1500):
+        p = S.make_problem(4, 12, 1, np.random.default_rng(1), compress=False)
+        p.states, p.freq, p.nptn = np.repeat(p.states, nptn, 1), np.ones(nptn), nptn
+        before = rec.rec_bytes()
+        t = G.Tree(p, all_directions=2)
+        t.full_traversal()
+        inner = [(u, int(v)) for u in range(12, 22) for v in p.nei[u] if v > u]
+        sizes = [rec.rec_bytes()]
+        for f in (t.all_branch_derivs, lambda: t.nni_evaluate(inner)):
+            called(f)
+            sizes.append(rec.rec_bytes())
+        t.close()
+        out.append((nptn // 64, len(inner), [b - a for a, b in zip(sizes, sizes[1:])], rec.rec_bytes() - before))
+    print(json.dumps(out))
+    """)
+    for tiles, moves, (derivs, nni), left in got:
+        slack = 1 << 20  # parameters, queued ops and their P(t)
+        assert derivs <= 2 * 12 * 32 * tiles + slack, (tiles, derivs)
+        assert nni <= (2 * moves * 144 * tiles if tiles <= 1024 else 0) + slack, (tiles, nni)
+        assert left == 0
