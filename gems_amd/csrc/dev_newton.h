@@ -22,11 +22,11 @@
 // writes the state to the host.
 //
 // A wait needs the branch's other workgroups on the device.  The launch rule (newton_solve_fits)
-// lets one branch take a quarter of the wavefront slots, and the workgroups of a branch are
-// neighbours in dispatch order, so the oldest unfinished branch always gets its slots once
-// earlier work drains.  Should they still not come (kernels of more than four queues that hold
-// each other's slots), a wait ends after NewtonState::wait and the workgroup leaves; the state stays
-// unfinished and the host solves with one launch per evaluation.
+// lets one branch take a quarter of the places (wavefront slots and LDS), and the workgroups of
+// a branch are neighbours in dispatch order, so the oldest unfinished branch always gets its
+// places once earlier work drains.  Should they still not come (kernels of more than four queues
+// that hold each other's places), a wait ends after NewtonState::wait and the workgroup leaves;
+// the state stays unfinished and the host solves with one launch per evaluation.
 #pragma once
 
 #include "dev_f64.h"
@@ -37,6 +37,14 @@ namespace dev {
 __device__ __forceinline__ double hand_empty() { return __longlong_as_double(-1ll); }
 __device__ __forceinline__ bool is_empty(double v) { return __double_as_longlong(v) == -1ll; }
 
+// A workgroup's LDS; MAXC: categories it has room for.
+template <int N, int MAXC, int K>
+struct NewtonLds {
+    double val[3][MAXC * N], cat[K][3][MAXC][64], inv[K][64], freq[K][64];
+    NewtonState st;
+    int sc[K][MAXC][64], go;
+};
+
 // L3: many-branch form (the logL of every evaluation, and one more evaluation at the answer where
 // bisection ended on an older point).  THETA: the products are read from P.theta instead of
 // formed from the partials at the branch.  hand: 3 NV ntiles empty places; spare: the places that
@@ -46,13 +54,13 @@ __device__ inline void newton_solve_body(const KParams &P, const int wg, const N
                                          double *spare, int64_t spare_len, NewtonState *out) {
     constexpr int NV = L3 ? 3 : 2;
     const int lane = threadIdx.x & 63, c = wave_id(), ncat = P.ncat;
-    const int nwg = (P.ntiles + K - 1) / K;
-    __shared__ double s_val[3][MAXC * N];
-    __shared__ double s_cat[K][3][MAXC][64];
-    __shared__ int s_sc[K][MAXC][64];
-    __shared__ double s_inv[K][64], s_freq[K][64];
-    __shared__ NewtonState s_st;
-    __shared__ int s_go;
+    __shared__ NewtonLds<N, MAXC, K> s;
+    auto &s_val = s.val;
+    auto &s_cat = s.cat;
+    auto &s_sc = s.sc;
+    auto &s_inv = s.inv, &s_freq = s.freq;
+    auto &s_st = s.st;
+    auto &s_go = s.go;
     if (threadIdx.x == 0) s_st = start;
     const uint64_t wait = (uint64_t)start.wait;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < spare_len; i += (int64_t)gridDim.x * blockDim.x)

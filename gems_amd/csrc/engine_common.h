@@ -273,7 +273,7 @@ hipError_t f64_theta_eval(const KParams &p, int deriv, hipStream_t s);
 hipError_t newton_first(NewtonState *st, const double *result, hipStream_t s);
 hipError_t f64_theta_newton(const KParams &p, NewtonState *st, hipStream_t s);
 // A whole solve per launch (dev_newton.h), while one branch's workgroups take at most a quarter of the
-// wavefront slots (four hardware queues can hold such launches side by side).
+// places on the device (four hardware queues can hold such launches side by side).
 bool newton_solve_fits(int n, int ncat, int ntiles, int ncu);
 // A finished state goes to *out (mapped host memory), an unfinished one (out->done unchanged) is left
 // to the per-evaluation launches.  hand: newton_hand_len doubles per branch, of all-ones bytes.

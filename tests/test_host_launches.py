@@ -120,3 +120,33 @@ def test_exchange_places_are_allocated_for_solves_only():
         assert derivs <= 2 * 12 * 32 * tiles + slack, (tiles, derivs)
         assert nni <= (2 * moves * 144 * tiles if tiles <= 1024 else 0) + slack, (tiles, nni)
         assert left == 0
+
+
+@pytest.mark.skipif(not os.path.exists(R.READELF), reason="llvm-readelf not available")
+@pytest.mark.parametrize("n", [4, 20, 61])
+def test_a_solve_takes_a_quarter_of_the_places(n):
+    """The workgroups of one branch wait for each other: four solves of different streams must fit the
+    256 compute units together, by wavefronts (16 a compute unit, 61 states 8) and by LDS."""
+    got = R.run(f"""
+    out, n = [], {n}
+    for ncat in range(1, 9):
+        for tiles in (1, 15, 64, 100, 128, 129, 255, 256, 257, 400, 512, 513, 700, 1024, 1025, 2047, 2048, 4096, 4097):
+            p = S.make_problem(n, 4, 1, np.random.default_rng(1), ncat=ncat, compress=False)
+            p.nptn = 64 * tiles
+            p.states, p.freq = np.repeat(p.states, p.nptn, 1), np.ones(p.nptn)
+            t = G.Tree(p, all_directions=2)
+            rec.rec_finish(1)
+            called(t.optimize_one, 0, int(p.nei[0, 0]))
+            called(t.nni_evaluate, [(4, 5)])
+            out.append((ncat, tiles, [k for k in launches() if "newton_solve" in k[0]]))
+            t.close()
+    print(json.dumps(out))
+    """)
+    static, seen = R.static_lds(), 0
+    for ncat, tiles, solves in got:
+        for name, _, blocks in solves:
+            places = min(LDS // static[name], (8 if n == 61 else 16) // ncat) * 256
+            blocks //= 2 if "multi" in name else 1  # two moves of one branch
+            assert 4 * blocks <= places, (ncat, tiles, name, blocks, places)
+            seen += 1
+    assert seen > 100
