@@ -100,6 +100,7 @@ _SIGS = {
     "plk_set_tile_shape": (_int, [_P, _int]),
     "plk_set_level_waves": (_int, [_P, _int]),
     "plk_set_solve_wait": (_int, [_P, _int]),
+    "plk_get_solve_counts": (_int, [_P, _i64p, _i64p]),
     "plk_set_f64_form": (_int, [_P, _int]),
     "plk_get_pattern_lh_cat": (_int, [_P, _dp]),
     "plk_get_pattern_scaling": (_int, [_P, _dp, _dp]),

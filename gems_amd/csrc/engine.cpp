@@ -1217,6 +1217,7 @@ extern "C" int plk_newton_branch(plk_ctx *c, int a, int b, double x1, double xgu
         c->theta_valid = true;
         c->theta_a = a;
         c->theta_b = b;
+        (h.done ? c->solves_one : c->solves_ended)++;
         if (h.done) {
             timing_collect(*c, used);
             return newton_result(h, out, evals);
@@ -1353,8 +1354,11 @@ extern "C" int plk_newton_multi(plk_ctx *c, int nbr, const int *a, const int *b,
                                       c->h_mnewton_dev, nbr, c->stream);
         }));
         HIP_TRY(hipStreamSynchronize(c->stream));
-        finished = true;
-        for (int i = 0; i < nbr && finished; i++) finished = h[i].done != 0;
+        int done = 0;
+        for (int i = 0; i < nbr; i++) done += h[i].done != 0;
+        c->solves_one += done;
+        c->solves_ended += nbr - done;
+        finished = done == nbr;
         if (!finished) HIP_TRY(hipMemcpyAsync(c->d_mnewton, h, sizeof(NewtonState) * nbr, hipMemcpyHostToDevice, c->stream));
     }
     if (!finished) rc = run_rounds(eval_only ? 1 : max_nr);
@@ -1521,6 +1525,14 @@ extern "C" int plk_set_solve_wait(plk_ctx *c, int microseconds) {
     clear_error();
     if (!c || microseconds < 0 || microseconds > 1000000) return fail(PLK_ERR_ARG, "plk_set_solve_wait: bad arguments");
     c->solve_wait = 100 * microseconds;
+    return PLK_OK;
+}
+
+extern "C" int plk_get_solve_counts(plk_ctx *c, int64_t *one_launch, int64_t *ended) {
+    clear_error();
+    if (!c || !one_launch || !ended) return fail(PLK_ERR_ARG, "plk_get_solve_counts: null argument");
+    *one_launch = c->solves_one;
+    *ended = c->solves_ended;
     return PLK_OK;
 }
 

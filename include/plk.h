@@ -207,6 +207,8 @@ int plk_set_level_waves(plk_ctx *ctx, int slots);
  * 20,000 us, at most 1 s).  A solve whose wait ends goes on with one launch per evaluation and
  * gives the same result; 0 ends nearly every wait. */
 int plk_set_solve_wait(plk_ctx *ctx, int microseconds);
+/* Branch solves of this context that finished in one launch, and those whose wait ended. */
+int plk_get_solve_counts(plk_ctx *ctx, int64_t *one_launch, int64_t *ended);
 
 /* Kernel timing with HIP events recorded on the context's stream around every launch
  * of the partial-traversal kernel.  kind: 0 traversal, 1 P(t), 2 derivative. */
