@@ -656,6 +656,23 @@ static hipError_t with_hand(Ctx &c, HandAreas &a, int64_t len, F &&launch) {
     return e;
 }
 
+// Whether this call solves in one launch.
+static bool one_launch(Ctx &c) {
+    if (!newton_solve_fits(c.n, c.ncat, c.ntiles, c.ncu)) return false;
+    if (c.solve_skip == 0) return true;
+    c.solve_skip--;
+    return false;
+}
+// After a wait that ended (20 ms lost) the context pauses for 256 calls, which take about as long by
+// themselves, and for twice as many after each further one in a row: what holds the places
+// (more busy streams than hardware queues) mostly lasts.
+static void solves_done(Ctx &c, int finished, int ended) {
+    c.solves_one += finished;
+    c.solves_ended += ended;
+    c.solve_pause = ended == 0 ? 0 : std::min(std::max(256, 2 * c.solve_pause), 8192);
+    c.solve_skip = c.solve_pause;
+}
+
 extern "C" int64_t plk_memory_required(int nstates, int ncat, int ntaxa, int nptn, int nslots, int precision,
                                        int scaling) {
     int64_t pad = round_up(nptn, 64), block = (int64_t)nstates * ncat, rs = precision == PLK_FP64 ? 8 : 4;
@@ -1196,7 +1213,7 @@ extern "C" int plk_newton_branch(plk_ctx *c, int a, int b, double x1, double xgu
     p.br_b = b;
     p.br_len = h.rts;
     bool used[3] = {false, false, false};
-    if (newton_solve_fits(c->n, c->ncat, c->ntiles, c->ncu)) {
+    if (one_launch(*c)) {
         // The whole solve in one launch, which in the FP64 form also builds theta.  A branch of an
         // optimisation round (its op, the solve, the host), before and after: DNA 954 patterns 70.5 ->
         // 33.2 us, 4,783 68.6 -> 34.2, 28,686 90 -> 47; protein 1,941 87 -> 46, 9,027 94 ->
@@ -1217,7 +1234,7 @@ extern "C" int plk_newton_branch(plk_ctx *c, int a, int b, double x1, double xgu
         c->theta_valid = true;
         c->theta_a = a;
         c->theta_b = b;
-        (h.done ? c->solves_one : c->solves_ended)++;
+        solves_done(*c, h.done != 0, h.done == 0);
         if (h.done) {
             timing_collect(*c, used);
             return newton_result(h, out, evals);
@@ -1345,7 +1362,7 @@ extern "C" int plk_newton_multi(plk_ctx *c, int nbr, const int *a, const int *b,
             round = std::min(2 * round, 48);
         }
     };
-    const bool whole = c->prec == PLK_FP64 && newton_solve_fits(c->n, c->ncat, c->ntiles, c->ncu);
+    const bool whole = c->prec == PLK_FP64 && one_launch(*c);
     bool finished = false;
     if (whole) {
         // every solve in one launch; what did not finish goes on below
@@ -1356,8 +1373,7 @@ extern "C" int plk_newton_multi(plk_ctx *c, int nbr, const int *a, const int *b,
         HIP_TRY(hipStreamSynchronize(c->stream));
         int done = 0;
         for (int i = 0; i < nbr; i++) done += h[i].done != 0;
-        c->solves_one += done;
-        c->solves_ended += nbr - done;
+        solves_done(*c, done, nbr - done);
         finished = done == nbr;
         if (!finished) HIP_TRY(hipMemcpyAsync(c->d_mnewton, h, sizeof(NewtonState) * nbr, hipMemcpyHostToDevice, c->stream));
     }
@@ -1525,6 +1541,7 @@ extern "C" int plk_set_solve_wait(plk_ctx *c, int microseconds) {
     clear_error();
     if (!c || microseconds < 0 || microseconds > 1000000) return fail(PLK_ERR_ARG, "plk_set_solve_wait: bad arguments");
     c->solve_wait = 100 * microseconds;
+    c->solve_skip = c->solve_pause = 0;
     return PLK_OK;
 }
 

@@ -225,6 +225,7 @@ struct Ctx {
     NewtonState *d_newton = nullptr, *h_newton = nullptr;  // device state, pinned host mirror
     NewtonState *h_newton_dev = nullptr;                   // the mirror's device address
     int solve_wait = 2000000;                              // NewtonState::wait: 20 ms
+    int solve_skip = 0, solve_pause = 0;                   // calls to go without one-launch solves; the last pause
     int64_t solves_one = 0, solves_ended = 0;              // one-launch solves that finished, whose waits ended
     HandAreas hand, mhand;                                 // exchange places of one-launch solves: one branch, many
     // host staging (pinned)

@@ -205,7 +205,9 @@ int plk_set_level_waves(plk_ctx *ctx, int slots);
 
 /* How long a workgroup of a one-launch Newton solve waits for the others of its branch (default
  * 20,000 us, at most 1 s).  A solve whose wait ends goes on with one launch per evaluation and
- * gives the same result; 0 ends nearly every wait. */
+ * gives the same result, and the context's next calls do so at once (256 of them, twice as
+ * many after each further ended wait in a row, until a one-launch solve finishes or this is
+ * set); 0 ends nearly every wait. */
 int plk_set_solve_wait(plk_ctx *ctx, int microseconds);
 /* Branch solves of this context that finished in one launch, and those whose wait ended. */
 int plk_get_solve_counts(plk_ctx *ctx, int64_t *one_launch, int64_t *ended);

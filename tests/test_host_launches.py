@@ -150,3 +150,29 @@ def test_a_solve_takes_a_quarter_of_the_places(n):
             assert 4 * blocks <= places, (ncat, tiles, name, blocks, places)
             seen += 1
     assert seen > 100
+
+
+def test_solves_whose_waits_end_are_not_tried_again_at_once():
+    """A solve whose wait ends has lost that time: the context goes back to one launch per evaluation
+    for a while, longer each time in a row, until a one-launch solve finishes or the bound is set."""
+    got = R.run("""
+    p = S.make_problem(4, 12, 300, np.random.default_rng(1), compress=False)
+    t = G.Tree(p)
+    w = int(p.nei[0, 0])
+    def tries(n, finish):
+        rec.rec_finish(finish)
+        for _ in range(n):
+            called(t.optimize_one, 0, w)
+        return sum("newton_solve" in k[0] for k in launches())
+    out = [tries(50, 1), tries(250, 0), tries(700, 0), tries(2000, 0), tries(8000, 1)]
+    tries(1, 0)
+    one, ended = ctypes.c_int64(), ctypes.c_int64()
+    G.lib().plk_get_solve_counts(t.context(), ctypes.byref(one), ctypes.byref(ended))
+    out += [one.value, ended.value]
+    G.lib().plk_set_solve_wait(t.context(), 20000)
+    out.append(tries(5, 1))
+    print(json.dumps(out))
+    """)
+    # pauses of 256, 512, 1,024 and 2,048 solves, one try between two of them; then 256 again
+    assert got[:5] == [50, 1, 2, 1, 8000 - 2048 + (50 + 250 + 700 + 2000) - (50 + 4 + 256 + 512 + 1024)]
+    assert got[5:] == [50 + got[4], 5, 5]
