@@ -129,9 +129,16 @@ hipError_t traverse_n(const KParams &p0, int mode, hipStream_t s) {
             // the op list on the matrix cores, then the branch stage alone (theta: no ops, in
             // the vector kernel)
             if (p.nops > 0) {
-                const int units = p.ntiles * (p.safe ? 4 * p.ncat : 16);
-                const dim3 g(std::min(units, 2 * std::max(1, p.ncu)));  // two stay on a compute unit
-                if (p.safe) hipLaunchKernelGGL(k_traverse_f64_codon<true>, g, dim3(256), 0, s, p);
+                // One category: the checks over a pattern and over a category are the same, and
+                // SAFE's workgroups have four wavefronts (NORM's one each left a compute unit two
+                // of eight: 20 taxa x 20,000 sites 452 us, now 218).
+                const bool safe = p.safe || p.ncat == 1;
+                const int units = p.ntiles * (safe ? 4 * p.ncat : 16);
+                // Workgroups that stay on a compute unit: eight wavefronts by registers, four
+                // workgroups by LDS (two categories 466 -> 321 us).
+                const int stay = safe ? 2 : std::min(4, 8 / p.ncat);
+                const dim3 g(std::min(units, std::max(1, stay * p.ncu)));
+                if (safe) hipLaunchKernelGGL(k_traverse_f64_codon<true>, g, dim3(256), 0, s, p);
                 else hipLaunchKernelGGL(k_traverse_f64_codon<false>, g, dim3(64 * p.ncat), 0, s, p);
                 if (mode == MODE_PARTIALS) return hipGetLastError();
                 p.nops = 0;

@@ -82,6 +82,7 @@ int rec_count() { return (int)g_launches.size(); }
 const char *rec_name(int i) { return g_launches[i].name.c_str(); }
 long rec_lds(int i) { return (long)g_launches[i].lds; }
 long rec_blocks(int i) { return (long)g_launches[i].grid.x * g_launches[i].grid.y; }
+long rec_threads(int i) { return (long)g_launches[i].block.x; }
 void rec_clear() { g_launches.clear(); }
 void rec_fail(const char *name) { g_fail = name; }
 void rec_finish(int on) { g_finish = on; }

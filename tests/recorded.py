@@ -15,7 +15,7 @@ PRELUDE = """
 import ctypes, json, sys
 sys.path[:0] = [{root!r}, {tests!r}]
 rec = ctypes.CDLL({stub!r}, mode=ctypes.RTLD_GLOBAL)
-for name in ("rec_lds", "rec_blocks", "rec_bytes"):
+for name in ("rec_lds", "rec_blocks", "rec_threads", "rec_bytes"):
     getattr(rec, name).restype = ctypes.c_long
 rec.rec_name.restype = ctypes.c_char_p
 import numpy as np

@@ -176,3 +176,27 @@ def test_solves_whose_waits_end_are_not_tried_again_at_once():
     # pauses of 256, 512, 1,024 and 2,048 solves, one try between two of them; then 256 again
     assert got[:5] == [50, 1, 2, 1, 8000 - 2048 + (50 + 250 + 700 + 2000) - (50 + 4 + 256 + 512 + 1024)]
     assert got[5:] == [50 + got[4], 5, 5]
+
+
+def test_codon_launch_fills_the_device():
+    """61 states in FP64: a long alignment gets as many workgroups as eight wavefronts a compute unit
+    hold, whatever the number of categories and the scaling."""
+    got = R.run("""
+    out = []
+    for ncat in range(1, 9):
+        for safe in (0, 1):
+            p = S.make_problem(61, 4, 1, np.random.default_rng(1), ncat=ncat, compress=False)
+            p.nptn = 64 * 400
+            p.states, p.freq = np.repeat(p.states, p.nptn, 1), np.ones(p.nptn)
+            t = G.Tree(p, scaling=safe)
+            called(t.full_traversal)
+            for i in range(rec.rec_count()):
+                if b"k_traverse_f64_codon" in rec.rec_name(i):
+                    out.append((ncat, safe, rec.rec_blocks(i) * rec.rec_threads(i) // 64))
+            rec.rec_clear()
+            t.close()
+    print(json.dumps(out))
+    """)
+    assert len(got) == 16
+    for ncat, safe, wavefronts in got:
+        assert wavefronts >= 256 * (8 if safe else 8 // ncat * ncat), (ncat, safe, wavefronts)
