@@ -359,6 +359,11 @@ enum : int { BATCH_MC = 0, BATCH_MC1 = 1, BATCH_20 = 2, BATCH_DNA = 3, BATCH_DNA
 constexpr int mc_batch_patterns(int ncat) { return 4 * mc_unit(ncat > 1 ? 2 : 1, ncat); }
 hipError_t batch_pmatrix_dna(int prec, const KParams *params, const PJob *jobs, int njobs, hipStream_t s);
 hipError_t batch_pmatrix(int prec, const KParams *params, const PJob *jobs, int njobs, hipStream_t s);
+// FP32 P(t) and traversals of BATCH_20 and BATCH_DNA in one launch each; kBothLds: at most the traversal's
+// own LDS arrays
+hipError_t batch_pmatrix_f32_both(const KParams *params, const PJob *jobs, int ndna, int njobs, hipStream_t s);
+hipError_t batch_traverse_f32_both(const KParams *params, const BatchItem *items, int nitems, size_t lds, hipStream_t s);
+constexpr size_t kBothLds = 20 * 1024;
 // lds: dynamic LDS of the BATCH_DNA launch
 hipError_t batch_traverse(int prec, int group, const KParams *params, const BatchItem *items, int nitems, int grid,
                           size_t lds, hipStream_t s);

@@ -19,14 +19,18 @@ __global__ void __launch_bounds__(256) k_batch_pmatrix_f64(const KParams *params
     pmatrix_f64_body(P, j);
 }
 
-__global__ void __launch_bounds__(256) k_batch_pmatrix_f32(const KParams *params, const PJob *jobs) {
-    const PJob j = load_uniform(jobs + blockIdx.x);
+__device__ __forceinline__ void pmatrix_f32_job(const KParams *params, const PJob *job) {
+    const PJob j = load_uniform(job);
     const KParams P = load_uniform(params + j.pad);
     switch (P.n) {
         case 4: pmatrix_f32_body<4>(P, j); break;
         case 20: pmatrix_f32_body<20>(P, j); break;
         default: break;
     }
+}
+
+__global__ void __launch_bounds__(256) k_batch_pmatrix_f32(const KParams *params, const PJob *jobs) {
+    pmatrix_f32_job(params, jobs + blockIdx.x);
 }
 
 // One kernel per state count: a kernel with both bodies takes the registers and LDS of the
@@ -55,8 +59,7 @@ __global__ void __launch_bounds__(256) k_batch_traverse_f64(const KParams *param
 
 // one thread per (job, category, state); batched partitions have at most four categories
 template <int FORM>
-__global__ void __launch_bounds__(256) k_batch_pmatrix_dna(const KParams *params, const PJob *jobs, int njobs) {
-    const int idx = blockIdx.x * 256 + threadIdx.x;
+__device__ __forceinline__ void pmatrix_dna_thread(const KParams *params, const PJob *jobs, int njobs, int idx) {
     if (idx >= njobs * 16) return;
     const PJob j = jobs[idx >> 4];
     const KParams &P = params[j.pad];
@@ -64,6 +67,18 @@ __global__ void __launch_bounds__(256) k_batch_pmatrix_dna(const KParams *params
     if (c >= P.ncat) return;
     dna_real<FORM> *M = (dna_real<FORM> *)P.mats + (int64_t)j.op * P.mat_stride + j.side * dna_side_len(FORM, 1);
     dna_pmat<FORM>(P, c, i, j.len, M, j.leaf ? M + dna_p_len(FORM) : nullptr);
+}
+
+template <int FORM>
+__global__ void __launch_bounds__(256) k_batch_pmatrix_dna(const KParams *params, const PJob *jobs, int njobs) {
+    pmatrix_dna_thread<FORM>(params, jobs, njobs, blockIdx.x * 256 + threadIdx.x);
+}
+
+// FP32 P(t) of both data types: nother workgroups, a job each, then those of the ndna jobs at
+// the head of the list
+__global__ void __launch_bounds__(256) k_batch_pmatrix_f32_both(const KParams *params, const PJob *jobs, int ndna, int nother) {
+    if ((int)blockIdx.x < nother) pmatrix_f32_job(params, jobs + ndna + blockIdx.x);
+    else pmatrix_dna_thread<1>(params, jobs, ndna, (blockIdx.x - nother) * 256 + threadIdx.x);
 }
 
 template <int FORM, bool SAFE, bool TURNS>
@@ -87,6 +102,15 @@ __global__ void __launch_bounds__(256) k_batch_traverse_f32(const KParams *param
     each_item<TURNS>(params, items, nitems, [&](const KParams &P, int tile) {
         if constexpr (N == 4) traverse_f32_valu_body<4, MODE_LOGL>(P, tile);
         else traverse_f32_mfma_body<N, MODE_LOGL>(P, tile);
+    });
+}
+
+// FP32, both data types (batch_traverse_f32_both)
+__global__ void __launch_bounds__(256) k_batch_traverse_f32_both(const KParams *params, const BatchItem *items, int nitems) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    each_item<false>(params, items, nitems, [&](const KParams &P, int tile) {
+        if (P.n == 20) traverse_f32_mfma_body<20, MODE_LOGL>(P, tile);
+        else traverse_dna_body<1, 1, MODE_LOGL, false, false>(P, tile, 0, P.nops, smem);
     });
 }
 
@@ -179,6 +203,19 @@ hipError_t batch_pmatrix(int prec, const KParams *params, const PJob *jobs, int 
     if (njobs <= 0) return hipSuccess;
     if (prec == PLK_FP64) hipLaunchKernelGGL(k_batch_pmatrix_f64, dim3(njobs), dim3(256), 0, s, params, jobs);
     else hipLaunchKernelGGL(k_batch_pmatrix_f32, dim3(njobs), dim3(256), 0, s, params, jobs);
+    return hipGetLastError();
+}
+
+hipError_t batch_pmatrix_f32_both(const KParams *params, const PJob *jobs, int ndna, int njobs, hipStream_t s) {
+    const int nother = njobs - ndna;
+    const dim3 grid(nother + (ndna * 16 + 255) / 256);
+    hipLaunchKernelGGL(k_batch_pmatrix_f32_both, grid, dim3(256), 0, s, params, jobs, ndna, nother);
+    return hipGetLastError();
+}
+
+hipError_t batch_traverse_f32_both(const KParams *params, const BatchItem *items, int nitems, size_t lds, hipStream_t s) {
+    if (lds + kBothLds > 160 * 1024) return hipErrorInvalidConfiguration;
+    hipLaunchKernelGGL(k_batch_traverse_f32_both, dim3(nitems), dim3(256), lds, s, params, items, nitems);
     return hipGetLastError();
 }
 

@@ -67,3 +67,23 @@ def test_batch_graph_replay_and_autotune():
     v2, _ = batch.loglik(br)
     alone2 = [t.loglik(*b) for t, b in zip(trees, br)]
     assert np.array_equal(v2, np.array(alone2))
+
+
+@pytest.mark.parametrize("tiles", [1, 3, 254, 256], ids=lambda t: f"{t}tiles")
+def test_fp32_both_data_types(tiles):
+    """FP32 DNA and protein partitions up to the item count (2 a compute unit, 512) that one launch
+    takes and past it: equal to the contexts alone, for graph replays and a given grid too."""
+    rng = np.random.default_rng(tiles)
+    probs = [S.make_problem(n, taxa, nptn, rng, ncat=ncat, ambiguous=0.03, compress=False)
+             for n, taxa, nptn, ncat in [(4, 9, 64 * tiles - 1, 4), (20, 9, 64 * tiles, 2), (4, 70, 65, 1), (20, 12, 1, 4)]]
+    say("batch fp32 both", tiles)
+    trees = [G.Tree(p, precision=G.FP32) for p in probs]
+    alone = np.array([t.full_traversal() for t in trees])
+    batch = G.Batch(trees)
+    br = [(0, int(p.nei[0, 0])) for p in probs]
+    for grid, graph in ((0, True), (0, True), (0, False), (64, True), (0, True)):
+        batch.set_launch(grid=grid, use_graph=graph)
+        for _ in range(2):
+            vals, _ = batch.loglik(br, clear=True)
+            assert np.array_equal(vals, alone), (grid, graph)
+    batch.close()

@@ -200,3 +200,23 @@ def test_codon_launch_fills_the_device():
     assert len(got) == 16
     for ncat, safe, wavefronts in got:
         assert wavefronts >= 256 * (8 if safe else 8 // ncat * ncat), (ncat, safe, wavefronts)
+
+
+def test_small_mixed_batch_is_two_launches():
+    """FP32 partitions of both data types whose items the device takes at once: one P(t) launch, one
+    traversal (more items: one of each per kernel)."""
+    got = R.run("""
+    out = []
+    for sizes in ((300, 200, 64), (64 * 255, 64 * 257), (64 * 256, 64 * 257), (300,)):
+        trees = []
+        for i, nptn in enumerate(sizes):
+            p = S.make_problem(20 if i == 0 and len(sizes) > 1 else 4, 5, nptn, np.random.default_rng(i), compress=False)
+            trees.append(G.Tree(p, precision=G.FP32))
+        b = G.Batch(trees)
+        launches()
+        rc = called(b.loglik, [(0, int(t.p.nei[0, 0])) for t in trees], clear=True)
+        out.append((rc, [n for n, _, _ in launches() if "pmatrix" in n or "traverse" in n]))
+        b.close()
+    print(json.dumps(out))
+    """)
+    assert [(rc, len(k)) for rc, k in got] == [(0, 2), (0, 2), (0, 4), (0, 2)], got
