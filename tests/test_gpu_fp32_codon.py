@@ -23,3 +23,21 @@ def test_units_match_whole_tiles(ncat, nptn):
         g.set_tile_shape(0)
         assert g.full_traversal() == v
     g.close()
+
+
+@pytest.mark.parametrize("ncat", [1, 4, 8])
+def test_few_jobs_give_the_same_matrices(ncat):
+    """P(t) of a few ops at a time (a workgroup per 16 rows) and of the whole list (matrix cores)
+    are equal to the bit."""
+    p = S.make_problem(61, 40, 30, np.random.default_rng(ncat), ncat=ncat, mean_len=0.2, ambiguous=0.05, compress=False)
+    print("61 states fp32 P(t)", ncat, flush=True)
+    g = G.Tree(p, precision=G.FP32)
+    v = g.full_traversal()
+    for u in range(40, 78, 9):
+        w = int(p.nei[u, 0])
+        t = g.get_length(u, w)
+        g.set_length(u, w, 2 * t)
+        assert g.compute_likelihood() != v
+        g.set_length(u, w, t)
+        assert g.compute_likelihood() == v
+    g.close()
