@@ -55,11 +55,12 @@ def run(code):
 
 
 @functools.lru_cache(maxsize=None)
-def static_lds():
-    """Kernel name -> bytes of its own LDS arrays, from the notes of the device code built here."""
+def kernel_notes():
+    """Kernel name -> (bytes of its own LDS arrays, vector registers), from the notes of the device
+    code built here."""
     with open(os.path.join(ROOT, "gems_amd", "libplk.so"), "rb") as f:
         data = f.read()
-    magic, sizes, at = b"__CLANG_OFFLOAD_BUNDLE__", {}, -1
+    magic, found, at = b"__CLANG_OFFLOAD_BUNDLE__", {}, -1
     while (at := data.find(magic, at + 1)) >= 0:
         pos = at + len(magic) + 8
         for _ in range(struct.unpack_from("<Q", data, at + len(magic))[0]):
@@ -69,11 +70,18 @@ def static_lds():
                     elf.write(data[at + off:at + off + size])
                     elf.flush()
                     notes = subprocess.run([READELF, "--notes", elf.name], check=True, capture_output=True, text=True).stdout
-                lds = None
+                kernel = {}
                 for line in notes.split("\n"):
-                    if ".group_segment_fixed_size:" in line:
-                        lds = int(line.split()[-1])
-                    elif line.startswith("    .name:") and lds is not None:
-                        sizes[line.split()[-1]] = lds
+                    if line.startswith("  - "):
+                        kernel = {}
+                    if line.startswith(("    .", "  - .")):
+                        key, _, value = line[4:].partition(":")
+                        kernel[key] = value.strip()
+                    if line.startswith("    .wavefront_size:"):
+                        found[kernel[".name"]] = int(kernel[".group_segment_fixed_size"]), int(kernel[".vgpr_count"])
             pos += 24 + length
-    return sizes
+    return found
+
+
+def static_lds():
+    return {name: lds for name, (lds, _) in kernel_notes().items()}

@@ -220,3 +220,11 @@ def test_small_mixed_batch_is_two_launches():
     print(json.dumps(out))
     """)
     assert [(rc, len(k)) for rc, k in got] == [(0, 2), (0, 2), (0, 4), (0, 2)], got
+
+
+@pytest.mark.skipif(not os.path.exists(R.READELF), reason="llvm-readelf not available")
+def test_fp32_derivative_kernels_leave_room_for_two_wavefronts():
+    """20 states: 256 vector registers at most (matrices read ahead of the category loop took 280)."""
+    kernels = {n: v for n, (_, v) in R.kernel_notes().items()
+               if any(k in n for k in ("k_multi_derivs_f32ILi20E", "k_multi_newtonILi20ELb1E", "k_theta_f32ILi20E"))}
+    assert len(kernels) == 3 and max(kernels.values()) <= 256, kernels
