@@ -883,7 +883,7 @@ __device__ inline bool theta_f32_body(const KParams &P, const int tile) {
         // values of 20 states went to lanes of registers ahead of the loop, and 280 registers left
         // one wavefront a SIMD.  NNI moves of 40 taxa x 4,000 sites 13.2 -> 6.4 ms, derivatives of
         // all branches 834 -> 587 us.
-        asm volatile("" : "+s"(piU), "+s"(uinv));
+        if constexpr (N == 20) asm volatile("" : "+s"(piU), "+s"(uinv));
         const int64_t off = ((int64_t)tile * ncat + c) * N * 64 + lane;  // theta (FP64 layout)
         const int64_t offf = ((int64_t)tile * ncat + c) * N * 64 + f32_loff(N, lane);
         double a[N], b[N];
