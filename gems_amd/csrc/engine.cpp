@@ -548,7 +548,8 @@ static int run_traversal(Ctx &c, KParams &p, int mode, bool used[3]) {
             HIP_TRY(hipMemcpyAsync(c.d_jobs, h + ob + xb, jb, hipMemcpyHostToDevice, c.stream));
             timing_begin(c, 1);
             if (dna) HIP_TRY(dna_pmatrix(p, f32 ? 1 : 0, c.d_jobs, njobs, c.stream));
-            else HIP_TRY(f32 ? f32_pmatrix(p, c.d_jobs, njobs, c.stream) : f64_pmatrix(p, c.d_jobs, njobs, c.stream));
+            else if (f32) HIP_TRY(f32_pmatrix(p, c.d_jobs, njobs, std::any_of(c.jobs.begin(), c.jobs.end(), [](const PJob &j) { return j.leaf; }), c.stream));
+            else HIP_TRY(f64_pmatrix(p, c.d_jobs, njobs, c.stream));
             timing_end(c, 1);
             used[1] = true;
         }

@@ -284,7 +284,8 @@ hipError_t newton_solve(const KParams &p, bool from_theta, const NewtonState &st
                         hipStream_t s);
 hipError_t newton_solve_multi(int n, int ncat, int ntiles, const KParams *params, const NewtonState *start,
                               HandArea hand, NewtonState *states, int nbr, hipStream_t s);
-hipError_t f32_pmatrix(const KParams &p, const PJob *jobs, int njobs, hipStream_t s);
+// leaf: some job forms a leaf table
+hipError_t f32_pmatrix(const KParams &p, const PJob *jobs, int njobs, bool leaf, hipStream_t s);
 hipError_t f32_traverse(const KParams &p, int mode, hipStream_t s);
 hipError_t f32_theta(const KParams &p, hipStream_t s);
 // level-parallel 4-state traversal (form 0 FP64, 1 FP32), lds_bytes of dynamic LDS

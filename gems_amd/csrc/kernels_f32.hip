@@ -155,7 +155,7 @@ hipError_t traverse_f32_n(const KParams &p, int mode, hipStream_t s) {
 
 }  // namespace
 
-hipError_t f32_pmatrix(const KParams &p, const PJob *jobs, int njobs, hipStream_t s) {
+hipError_t f32_pmatrix(const KParams &p, const PJob *jobs, int njobs, bool leaf, hipStream_t s) {
     switch (p.n) {
         case 4: hipLaunchKernelGGL(k_pmatrix_f32<4>, dim3(njobs * p.ncat), dim3(256), 0, s, p, jobs); break;
         case 20:
@@ -163,8 +163,9 @@ hipError_t f32_pmatrix(const KParams &p, const PJob *jobs, int njobs, hipStream_
             break;
         case 61:
             // The same values from either kernel.  A few jobs are their latency: a workgroup per 16
-            // rows while every one has a compute unit to itself (37 jobs, one category: 20.3 us against 27.7).
-            if (4 * njobs * p.ncat <= p.ncu)
+            // rows while every one has a compute unit to itself (37 jobs, one category: 20.3 us against
+            // 27.7), but not without leaf tables, which are most of that chain (54 us a call against 51).
+            if (leaf && 4 * njobs * p.ncat <= p.ncu)
                 hipLaunchKernelGGL(k_pmatrix_f32<61>, dim3(njobs * p.ncat * f32_xblocks(61)), dim3(256), 0, s, p, jobs);
             else
                 hipLaunchKernelGGL(k_pmatrix_f32_codon, dim3(njobs * p.ncat), dim3(256), 0, s, p, jobs);
