@@ -39,8 +39,9 @@ __device__ __forceinline__ bool is_empty(double v) { return __double_as_longlong
 
 // A workgroup's LDS; MAXC: categories it has room for.
 template <int N, int MAXC, int K>
-struct NewtonLds {
-    double val[3][MAXC * N], cat[K][3][MAXC][64], inv[K][64], freq[K][64];
+struct alignas(16) NewtonLds {
+    alignas(16) double val[3][MAXC * N];
+    double cat[K][3][MAXC][64], inv[K][64], freq[K][64];
     NewtonState st;
     int sc[K][MAXC][64], go;
 };
