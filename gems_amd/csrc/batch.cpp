@@ -1,7 +1,8 @@
 // Batched unlinked partitions: many contexts (one per partition, like the per-partition
-// PhyloTrees of PhyloSuperTree, tree/phylosupertree.cpp:662-734) evaluated with one P(t)
-// launch and one persistent traversal launch, replayed as a HIP graph while the launch
-// shape is unchanged, with the persistent grid chosen by a measuring autotuner.
+// PhyloTrees of PhyloSuperTree, tree/phylosupertree.cpp:662-734) evaluated with a P(t) and a
+// traversal launch per kernel (4 states, 20 states; one of each for a small FP32 batch of
+// both), replayed as a HIP graph while the launch shape is unchanged; the autotuner measures
+// grids whose workgroups take items in turns.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -4,8 +4,9 @@
 // workgroup owns one tile and its wavefronts split the categories (wave w handles
 // c = w, w + nwaves, ...).  Element (ptn, c, x) of a partial is at
 // ((tile*ncat + c)*n + x)*64 + lane, so every load/store of one (c, x) by a wavefront
-// is one contiguous 512-byte segment (20 states: eight 64-byte ones, 61: sixteen 32-byte ones, see f64_xoff).  All tiles are independent across the whole
-// traversal (the reference's packets walk every node for their pattern slice,
+// is one contiguous 512-byte segment (20 states: eight 64-byte ones, 61: sixteen 32-byte
+// ones, see f64_xoff).  All tiles are independent across the whole traversal (the
+// reference's packets walk every node for their pattern slice,
 // tree/phylokernelnew.h:2851-2853), so one launch runs the full post-order op list with
 // no grid-wide barrier; each thread only re-reads values it wrote itself.
 #pragma once
@@ -17,8 +18,8 @@ namespace dev {
 
 // ---------------------------------------------------------------------------------------
 // P(t) kernel (computePartialInfo, tree/phylokernelnew.h:1013-1063): for one child of one
-// op, echild[c][x][i] = U[x][i] exp(lambda_i r_c t) (held as [c][i][x] for n <= 20), and
-// for a leaf child the table
+// op, echild[c][x][i] = U[x][i] exp(lambda_i r_c t) (held as [c][i][x]; the matrix-core
+// traversals take the exponentials alone), and for a leaf child the table
 // leaf[s][c][x] = sum_i echild[c][x][i] tip_lh[s][i] with the unknown-state row = 1.
 // ---------------------------------------------------------------------------------------
 // 61-state (codon) op with its matrices in LDS.  A 61-double column does not fit the

@@ -5,8 +5,9 @@
 //   a = E_L L,  b = E_R R  (E = U diag(exp(Lambda r t))),  out = U^-1 (a o b)
 // with tip children replaced by leaf-table rows (1729-1747, 1848-1890).  Written as
 // a = U (exp(Lambda r t) o L), the matrices are U and U^-1 for every op, side and category, so
-// they stay in registers for the whole launch and an op reads only its children's rows
-// and 20 exponentials per side and category (reading E instead, 12.8 KB per side and
+// they are in LDS for the whole launch (read anew in each product: in registers they would
+// take 50 each) and an op reads from memory only its children's rows and 20 exponentials
+// per side and category (reading E instead, 12.8 KB per side and
 // wavefront, kept the vector L1 busy 70 % of the time: 1.60 ms for 100 taxa x 49,994
 // patterns).
 //

@@ -1,5 +1,5 @@
 // FP64 traversal of 61-state models on the matrix cores: a wavefront takes four patterns of
-// one category through the op list, with both constant matrices in its registers.
+// one category through the op list, with U in its registers and U^-1 in LDS.
 //
 // Per op and category the eigen-space partial (tree/phylokernelnew.h:1911-2036) is
 //   a = U (exp(Lambda r t_L) o L),  b alike,  out = U^-1 (a o b)

@@ -37,7 +37,8 @@ static int64_t round_up(int64_t v, int64_t g) { return (v + g - 1) / g * g; }
 static bool supported_states(int n) { return n == 4 || n == 20 || n == 61; }
 
 // per-op matrix block (in reals): transition data for both children + leaf tables for
-// both children.  FP64: echild[c][x][i]; FP32: matrix-core fragments of P_c.
+// both children.  FP64: the exponentials (matrix-core traversals) or echild[c][i][x]; FP32:
+// P_c, as matrix-core fragments for 20 and 61 states.
 static int64_t mat_stride_of(int n, int ncat, int su, int prec) {
     if (prec == PLK_FP32) {
         int64_t fr = (int64_t)f32_xblocks(n) * f32_ksteps(n) * 64;

@@ -154,7 +154,7 @@ struct KParams {
     int br_lds_a, br_lds_b;   // LDS buffer (or staged tip index) of the branch's two sides
     int small_stage;          // level-parallel kernel: op list, level bounds and P(t) exponentials staged in LDS;
                               // dev_dna.h: ops whose P(t) data a workgroup stages at most
-    const double *uinv_frag;  // FP64 matrix-core traversal: U^-1 as A fragments (null: not built)
+    const double *uinv_frag;  // FP64 matrix-core traversals: U and U^-1 in the kernels' order (mfma64_uinv_frag_size)
     int f64_form;             // FP64 20/61 states: 1 matrix-core traversal, 0 vector-ALU kernels
 };
 
@@ -240,9 +240,9 @@ struct Ctx {
     bool ptn_lh_valid = false;  // d_ptn_lh holds the per-pattern logL of the last logL evaluation
     bool timing = false;
     int wpc = 1;  // FP32 matrix-core tile shape (plk_set_tile_shape)
-    double *d_uinv_frag = nullptr;  // FP64 20/61 states: U^-1 as matrix-core fragments
-    int f64_form = -1;              // FP64 20/61 states, ncat <= 4: 1 matrix cores, 0 vector ALU,
-                                    // -1 by state count (61: matrix cores, 20: vector ALU)
+    double *d_uinv_frag = nullptr;  // FP64 20/61 states: U and U^-1 for the matrix cores
+    int f64_form = -1;              // FP64 20/61 states: 1 matrix cores, 0 vector ALU, -1 the faster one
+                                    // (matrix cores for both, f64_form_of)
     // 4-state models: ops per level run at once by the level-parallel kernel (0: the
     // category-split kernels; -1: the traversal of dev_dna.h)
     int small_waves = -1;

@@ -1,9 +1,9 @@
 // Batched unlinked partitions (IQ-TREE's PhyloSuperTree loop over partitions,
-// tree/phylosupertree.cpp:662-734) in one launch per traversal: every work item is one
-// 64-pattern tile of one partition; each partition keeps its own model, P(t), slots,
-// scale counters and fixed-order reduction, so its result is bit-identical to running
-// it alone.  DNA and protein partitions share the launch (the state count is a
-// per-item branch, uniform within a workgroup).
+// tree/phylosupertree.cpp:662-734): a traversal is one launch per kernel (4 and 20 states
+// each have their own; a small FP32 batch of both is one launch), and every work item is
+// one workgroup's patterns of one partition.  Each partition keeps its own model, P(t),
+// slots, scale counters and fixed-order reduction, so its result is bit-identical to
+// running it alone.
 #include "dev_dna.h"
 #include "dev_f32.h"
 #include "dev_f64.h"

@@ -23,8 +23,10 @@
  *   - Partials use IQ-TREE's eigen-space representation in the FP64 form
  *     (tree/phylokernelnew.h:1989-1994) and are laid out on the device like the
  *     reference's SIMD layout with 64 lanes: element (ptn, c, x) at
- *     (floor(ptn/64)*block + c*n + x)*64 + ptn%64, block = ncat*n (20 states: inside the
- *     64-pattern block of a category, groups of 8 patterns, see f64_xoff/f64_loff).
+ *     (floor(ptn/64)*block + c*n + x)*64 + ptn%64, block = ncat*n (inside the 64-pattern
+ *     block of a category, 20 states: groups of 8 patterns, 61: of 4, see f64_xoff/f64_loff;
+ *     FP32 form, 4 states: the four states of a pattern together, 20: four at a time, see
+ *     f32_xoff/f32_loff).
  *   - scale counts follow scale_num (tree/phylonode.h:17, uint16): one per pattern in
  *     NORM mode, one per (pattern, category) in SAFE mode
  *     (tree/phylokernelnew.h:1924-1936, mode rule tree/phylotreesse.cpp:95-96).

@@ -3,11 +3,12 @@
  *
  * IQ-TREE evaluates a partitioned analysis by looping over per-partition PhyloTrees
  * (PhyloSuperTree::computeLikelihood, tree/phylosupertree.cpp:709-734, OpenMP over
- * partitions ordered by cost, :662-707).  A batch runs that loop as ONE P(t) launch plus
- * one persistent traversal launch per kernel (4 states, 20 states) over all partitions'
- * pattern tiles, replayed as a HIP graph while the launch shape is unchanged.  Each partition is a plk_ctx whose ops
- * were queued with plk_update_partials; results per partition are bit-identical to
- * evaluating that context alone.
+ * partitions ordered by cost, :662-707).  A batch runs that loop as one P(t) launch and one
+ * traversal launch per kernel (4 states, 20 states; a small FP32 batch of both as one of
+ * each) over all partitions' pattern tiles, replayed as a HIP graph while the launch shape
+ * is unchanged.  Each partition is a plk_ctx whose ops were queued with
+ * plk_update_partials; results per partition are bit-identical to evaluating that context
+ * alone.
  */
 #ifndef PLK_BATCH_H
 #define PLK_BATCH_H
