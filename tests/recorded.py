@@ -1,6 +1,7 @@
 """Runs a snippet against libplk.so with hip_record.cpp in the place of the HIP runtime, in a
 process of its own (CPU only)."""
 import functools
+import json
 import os
 import struct
 import subprocess
@@ -36,9 +37,12 @@ def called(f, *a, **k):
 """
 
 
+KEEP = tempfile.TemporaryDirectory()  # until the tests end
+
+
 @functools.lru_cache(maxsize=None)
 def stub():
-    out = os.path.join(tempfile.mkdtemp(), "hip_record.so")
+    out = os.path.join(KEEP.name, "hip_record.so")
     subprocess.run(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
                     "-I" + os.path.join(ROOT, "include"), "-I" + os.path.join(ROOT, "gems_amd", "csrc"),
                     os.path.join(ROOT, "tests", "hip_record.cpp"), "-o", out], check=True, timeout=300)
@@ -50,7 +54,6 @@ def run(code):
     text = PRELUDE.format(root=ROOT, tests=os.path.join(ROOT, "tests"), stub=stub()) + textwrap.dedent(code)
     r = subprocess.run([sys.executable, "-c", text], capture_output=True, text=True, timeout=600)
     assert r.returncode == 0, r.stderr[-2000:]
-    import json
     return json.loads(r.stdout.strip().split("\n")[-1])
 
 
